@@ -26,11 +26,16 @@ _int = ctypes.c_int
 _flt = ctypes.c_float
 
 
+def reference_present() -> bool:
+    """The reference's sources lie under /root/reference (the folder may also be empty)."""
+    return os.path.isfile("/root/reference/src/orionsbelt/engines/cpu/kernels/gdn_sve.c")
+
+
 def build() -> None:
     """Compile liborb_oracle.so (and oracle/_ref when the reference tree is
     present).  Raises CalledProcessError on a compiler error."""
     subprocess.run(["make", "-s", "-C", HERE, "all"], check=True)
-    if os.path.isdir("/root/reference"):
+    if reference_present():
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
