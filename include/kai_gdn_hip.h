@@ -287,10 +287,13 @@ int kai_run_gdn_w8a16_gemm_hip(const uint16_t *x, const int8_t *Wq, const float 
  * calls that share it must not overlap.  0 workspace bytes: none needed.
  * For M <= 3, N <= 32768 and K of 2560, 4096 or 9216 (the Qwen3.5-4B
  * matrices but the LM head) one 16-channel tile per block runs instead,
- * with no k-split; the workspace is then unused.  M > 16 (a prompt's rows: the counterpart of the reference
- * e2e loop's M > 1 gemm_int8_neon, gdn_e2e_decode.c:606-612) takes the
- * prefill GEMM on fp16 MFMA (128 x 128 output tiles below 512 rows, 256 x
- * 256 from 512), and no workspace. */
+ * with no k-split; the workspace is then unused.  M > 16 (a prompt's rows:
+ * the counterpart of the reference e2e loop's M > 1 gemm_int8_neon,
+ * gdn_e2e_decode.c:606-612) takes the prefill GEMM on fp16 MFMA (64, 128 or
+ * 256 x 256 output tiles).  Its workspace is optional and needs no zeroing:
+ * with the bytes that the query returns, few rows split k across blocks
+ * (summed in a fixed order); with less, or none, they split less or not at
+ * all.  It changes nothing of a workspace that a call with M <= 16 keeps. */
 int kai_run_gdn_w8_tile_hip(const int8_t *Wq, int8_t *Wt, int N, int K, void *stream);
 size_t kai_gdn_w8a16_gemm_tiled_workspace_bytes(int M, int N, int K);
 int kai_run_gdn_w8a16_gemm_tiled_hip(const uint16_t *x, const int8_t *Wt, const float *scale,

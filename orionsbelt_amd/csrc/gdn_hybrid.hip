@@ -466,7 +466,8 @@ struct kai_gdn_hybrid {
     uint32_t *gemm_cnt = nullptr;  // zero between launches
     // prefill buffers, allocated by the first prefill for max_context rows
     struct Prefill {
-        int rows = 0, tv = 0;  // capacity (positions) and the V^T row length
+        int rows = 0, tv = 0;   // capacity (positions) and the V^T row length
+        float *part = nullptr;  // k-split partials of the GEMMs, w8p_part_bytes_max() bytes
         float *h = nullptr, *qkv = nullptr, *z = nullptr, *a = nullptr, *b = nullptr;
         float *g = nullptr, *beta = nullptr, *kx = nullptr, *vx = nullptr, *hist = nullptr;
         uint16_t *x16 = nullptr, *act16 = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *o = nullptr;
@@ -870,20 +871,22 @@ hipError_t prefill_alloc(kai_gdn_hybrid *m) {
     TRY(alloc_t(m, &p.vT, (size_t)Hkv * 256 * p.tv));
     // V^T past a prefill's length is read (with weight 0): keep it finite
     TRY(hipMemset(p.vT, 0, (size_t)Hkv * 256 * p.tv * sizeof(uint16_t)));
+    TRY(alloc(m, reinterpret_cast<void **>(&p.part), w8p_part_bytes_max()));
     p.rows = (int)R;
     return hipDeviceSynchronize();
 }
 
-hipError_t w8p(const uint16_t *x, int ldx, const Mat &w, int M, const W8Out &o, hipStream_t st) {
-    return launch_w8p(x, ldx, w.q, w.s, M, w.N, w.K, o, st);
+hipError_t w8p(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, int M, const W8Out &o, hipStream_t st) {
+    return launch_w8p(x, ldx, w.q, w.s, M, M, M, w.N, w.K, o, m->pf.part, w8p_part_bytes_max(), st);
 }
 // A branch matrix: h[t] += x[t] W^T for the T rows, the residual add in the
 // GEMM's epilogue (in place), so no branch array is written and read back.
-hipError_t w8p_residual(const uint16_t *x, int ldx, const Mat &w, int M, float *h, int H, hipStream_t st) {
+hipError_t w8p_residual(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, int M, float *h, int H,
+                        hipStream_t st) {
     W8Out o = segments({{h, H, H}});
     o.add_in = h;
     o.add_ld = H;
-    return w8p(x, ldx, w, M, o, st);
+    return w8p(m, x, ldx, w, M, o, st);
 }
 
 // One sequence's prompt through every layer at once: T rows of sequence b.
@@ -906,7 +909,7 @@ hipError_t prefill_seq(kai_gdn_hybrid *m, const int32_t *tokens, int b, int T, h
     for (size_t l = 0; l < m->layers.size(); ++l) {
         Layer &L = m->layers[l];
         if (!L.attn) {
-            TRY(w8p(p.x16, H, L.in, T, segments({{p.qkv, C, C}, {p.z, V, C + V}, {p.b, Hv, C + V + Hv},
+            TRY(w8p(m, p.x16, H, L.in, T, segments({{p.qkv, C, C}, {p.z, V, C + V}, {p.b, Hv, C + V + Hv},
                                                   {p.a, Hv, C + V + 2 * Hv}}), st));
             TRY(mark(m, KAI_GDN_PHASE_GDN_PROJ, st));
             // the decode step's conv cache: the last four conv inputs
@@ -924,11 +927,11 @@ hipError_t prefill_seq(kai_gdn_hybrid *m, const int32_t *tokens, int b, int T, h
                                                                                   c.rms_eps);
             TRY(hipGetLastError());
             TRY(mark(m, KAI_GDN_PHASE_GDN_CORE, st));
-            TRY(w8p_residual(p.x16, V, L.out, T, p.h, H, st));
+            TRY(w8p_residual(m, p.x16, V, L.out, T, p.h, H, st));
             TRY(mark(m, KAI_GDN_PHASE_GDN_OPROJ, st));
         } else {
             const int nq = Hq * 512, nkv = Hkv * 256;
-            TRY(w8p(p.x16, H, L.in, T, segments({{p.qkv, nq, nq}, {p.kx, nkv, nq + nkv}, {p.vx, nkv, nq + 2 * nkv}}),
+            TRY(w8p(m, p.x16, H, L.in, T, segments({{p.qkv, nq, nq}, {p.kx, nkv, nq + nkv}, {p.vx, nkv, nq + 2 * nkv}}),
                     st));
             attn_prologue_rows_kernel<<<dim3((T + 4 * kApRows - 1) / (4 * kApRows), Hq + 2 * Hkv), 256, 0, st>>>(
                 p.qkv, p.kx, p.vx, L.q_norm, L.k_norm, p.q16, L.Kc, L.Vc, Hq, Hkv, m->tmax, T, b, c.rope_theta,
@@ -937,13 +940,13 @@ hipError_t prefill_seq(kai_gdn_hybrid *m, const int32_t *tokens, int b, int T, h
             const size_t kvrow = (size_t)b * Hkv * m->tmax * 256;
             TRY(launch_attn_prefill(p.q16, L.Kc + kvrow, p.vT, p.qkv + 256, nq, p.x16, T, Hq, Hkv, m->tmax, p.tv,
                                     1.0f / 16.0f, st));
-            TRY(w8p_residual(p.x16, Hq * 256, L.out, T, p.h, H, st));
+            TRY(w8p_residual(m, p.x16, Hq * 256, L.out, T, p.h, H, st));
             TRY(mark(m, KAI_GDN_PHASE_ATTN, st));
         }
         addnorm_kernel<<<T, 256, 0, st>>>(p.h, nullptr, L.ln_post, p.x16, H, c.rms_eps);
         TRY(hipGetLastError());
-        TRY(w8p(p.x16, H, L.gate_up, T, swiglu, st));
-        TRY(w8p_residual(p.act16, I, L.down, T, p.h, H, st));
+        TRY(w8p(m, p.x16, H, L.gate_up, T, swiglu, st));
+        TRY(w8p_residual(m, p.act16, I, L.down, T, p.h, H, st));
         const float *next_norm = l + 1 < m->layers.size() ? m->layers[l + 1].ln_in : m->final_norm;
         addnorm_kernel<<<T, 256, 0, st>>>(p.h, nullptr, next_norm, p.x16, H, c.rms_eps);
         TRY(hipGetLastError());

@@ -191,11 +191,18 @@ hipError_t launch_w8_quantize(const float *W, int8_t *Wq, float *scale, int N, i
 
 // The model's int8 GEMM for many rows: x [M][ldx] fp16 (16-byte aligned
 // rows), weights tiled by launch_w8f_tile (N % 64 == 0, K % 64 == 0); `out`
-// as for launch_w8f in kW8Segments or kW8SwiGLU mode.
-// The largest M launch_w8p accepts (its grid's y limit).
+// as for launch_w8f in kW8Segments or kW8SwiGLU mode.  The M rows are
+// sequences of seq_rows rows (M for one); row values depend on seq_rows and
+// max_rows (>= M), not on M.  `part` (may be null) holds part_bytes of
+// scratch for k-splits, uninitialised; with less than the best split needs, fewer
+// splits run.
+// The largest M launch_w8p accepts.
 long long w8p_max_rows();
-hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int N, int K,
-                      const W8Out &out, hipStream_t st);
+// Scratch the best split of M rows (one sequence) uses, and the most any uses.
+size_t w8p_part_bytes(int M, int N, int K);
+size_t w8p_part_bytes_max();
+hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
+                      int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st);
 // Causal attention of one sequence's T positions: q16 [T][Hq][256] fp16,
 // Kc [Hkv][Tmax][256] tiled by 16 positions (kv_tiled_offset), vT
 // [Hkv][256][Tv] fp16 (V transposed; Tv % 64 == 0, Tv >= T, finite past T),

@@ -4,18 +4,15 @@
 // Prefill GEMM: y[m][n] = scale[n] sum_k x[m][k] Wq[n][k] for M rows (a
 // whole prompt), on the same pre-tiled int8 weights as the decode GEMM
 // (gdn_model.hip, w8f_tile_kernel) -- the M > 1 counterpart of the
-// reference e2e loop's gemm_int8_neon (gdn_e2e_decode.c:606-612).  Block
-// tile 128 rows x 128 channels, k in steps of 64, 4 waves as 2 x 2 (64 x 64
-// each, four 32x32x16 fp16 MFMA tiles: the larger MFMA shape delivers about
-// 1.5 times the 16x16x32 rate on gfx950).  Per step a thread stages 4 x 16
-// bytes of activations and 2 x 16 bytes of weights in registers while the
-// waves multiply the previous step from LDS; the weights are widened to
-// fp16 (exactly) on their way into LDS, so every MFMA operand is one
-// 16-byte LDS read.  LDS rows are 64 k + 8 pad halves (144 bytes): the
-// 16-byte reads of 8 consecutive rows then cover the 32 banks once.  The
-// weight is the A operand, so a lane's accumulators hold runs of 4
-// consecutive channels of one row (16-byte stores), and the interleaved
-// gate/up rows put each gate channel and its up channel in the same lane.
+// reference e2e loop's gemm_int8_neon (gdn_e2e_decode.c:606-612).  Persistent
+// blocks of 64, 128 or 256 rows x 256 channels (w8t_kernel), k in steps of
+// 64, 32x32x16 fp16 MFMA (the larger MFMA shape delivers about 1.5 times the
+// 16x16x32 rate on gfx950); both operands reach LDS by DMA, the weights as
+// int8, widened to fp16 (exactly) on their way into the MFMA.  The weight is
+// the A operand, so a lane's accumulators hold runs of 4 consecutive channels
+// of one row, and the interleaved gate/up rows put each gate channel and its
+// up channel in the same lane.  Few rows leave most CUs without a tile: their
+// k-steps are split over blocks (w8t_choose).
 //
 // Prefill attention: Qwen3_5Attention's causal softmax(q k^T / 16) v with
 // the sigmoid output gate (modeling_qwen3_5.py:629-701), GQA, head dim 256,
@@ -29,324 +26,472 @@
 // score registers as the B operand (the 8 keys a lane holds, 4g .. 4g+3 and
 // 16 + 4g .. 16 + 4g+3, permute the k index of both operands alike).  Each K
 // and V fragment read from LDS feeds both query tiles.
+#include <algorithm>
+
 #include "gdn_common.h"
 #include "gdn_internal.h"
 
 namespace gdn {
 namespace {
 
-constexpr int kPBM = 128;    // activation rows per block
-constexpr int kPBN = 128;    // channels per block (two 64-channel groups of the tiled weights)
-constexpr int kPPitch = 72;  // halves per LDS row: 64 k + 8
-
-struct W8pStage {
-    uint16_t x[kPBM * kPPitch];
-    uint16_t w[kPBN * kPPitch];
-};
-
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-// Epilogue of one 32x32 accumulator tile (channels nt .. nt+31, one row per
-// lane): lane l holds, for q = 0..3, channels nt + 8 q + 4 (l / 32) .. +3 of
-// its row (C element 4 q + e).
-GDN_DEV void w8p_store_tile(const f32x16_t &acc, int row, int nt, int h2, const float *__restrict__ scale, int N,
-                            const W8Out &out) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int n = nt + 8 * q + 4 * h2;
-        const f32x4_t sc = *reinterpret_cast<const f32x4_t *>(scale + n);
-        f32x4_t y = f32x4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]} * sc;
-        if (out.mode == kW8SwiGLU) {
-            // 16-channel groups: 8 gate channels (q even), then their 8 up channels (q + 1)
-            if (q & 1) continue;
-            const f32x4_t su = *reinterpret_cast<const f32x4_t *>(scale + n + 8);
-            const f32x4_t up = f32x4_t{acc[4 * q + 4], acc[4 * q + 5], acc[4 * q + 6], acc[4 * q + 7]} * su;
-            uint32_t hv[2];
-#pragma unroll
-            for (int e = 0; e < 4; e += 2) {
-                const float a = y[e] / (1.0f + expf(-y[e])) * up[e];
-                const float b = y[e + 1] / (1.0f + expf(-y[e + 1])) * up[e + 1];
-                hv[e / 2] = (uint32_t)f32_to_f16_rne(a) | ((uint32_t)f32_to_f16_rne(b) << 16);
-            }
-            const int cc = (nt + 16 * (q >> 1)) / 2 + 4 * h2;
-            *reinterpret_cast<uint2 *>(out.x16 + (size_t)row * (N / 2) + cc) = make_uint2(hv[0], hv[1]);
-        } else if (n < out.seg[out.nseg - 1].n_end) {  // channels past the last segment: padding
-            int sgi = 0, nb = 0;
-#pragma unroll
-            for (int qq = 0; qq < kW8MaxSegs - 1; ++qq)
-                if (qq < out.nseg - 1 && n >= out.seg[qq].n_end) {
-                    sgi = qq + 1;
-                    nb = out.seg[qq].n_end;
-                }
-            float *dst = out.seg[0].dst;
-            int ld = out.seg[0].ld;
-#pragma unroll
-            for (int qq = 1; qq < kW8MaxSegs; ++qq)
-                if (qq == sgi) {
-                    dst = out.seg[qq].dst;
-                    ld = out.seg[qq].ld;
-                }
-            // the residual add (one segment): may be in place, each element
-            // is read and written by this lane only
-            if (out.add_in) y = *reinterpret_cast<const f32x4_t *>(out.add_in + (size_t)row * out.add_ld + n) + y;
-            *reinterpret_cast<f32x4_t *>(dst + (size_t)row * ld + (n - nb)) = y;
-        }
-    }
-}
-
-__global__ __launch_bounds__(256, 2) void w8p_kernel(const uint16_t *__restrict__ X, int ldx,
-                                                     const int8_t *__restrict__ W, const float *__restrict__ scale,
-                                                     int M, int N, int K, W8Out out) {
-    __shared__ __align__(16) W8pStage st[2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;  // rows 64 wm .., channels 64 wn .. of the block
-    const int n0 = blockIdx.x * kPBN, m0 = blockIdx.y * kPBM;
-    const int steps = K / 64;
-    const bool two = n0 + 64 < N;        // the block's second channel group exists
-    const bool active = wn == 0 || two;  // this wave's channels exist (wave-uniform)
-
-    // staging: activation chunk c = tid + 256 i is row c / 8, k 8 (c % 8) .. +7
-    // (rows past M read row M - 1, never stored); weight chunk tid of each
-    // group's 4 KB step block (tile tid / 64, tiled lane tid % 64)
-    const uint16_t *xp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int c = tid + 256 * i;
-        xp[i] = X + (size_t)min(m0 + (c >> 3), M - 1) * ldx + (c & 7) * 8;
-    }
-    const int8_t *wp0 = W + (size_t)(n0 / 64) * steps * 4096 + tid * 16;
-    const int8_t *wp1 = two ? wp0 + (size_t)steps * 4096 : wp0;
-    // Two register stages: the loads of step s + 2 are issued before the
-    // waves multiply step s, so each load has two steps' compute to land.
-    struct Stage {
-        u32x4_t x[4], w[2];
-    };
-    auto gload = [&](int s, Stage &r) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r.x[i] = *reinterpret_cast<const u32x4_t *>(xp[i] + s * 64);
-        r.w[0] = *reinterpret_cast<const u32x4_t *>(wp0 + (size_t)s * 4096);
-        r.w[1] = *reinterpret_cast<const u32x4_t *>(wp1 + (size_t)s * 4096);
-    };
-    const int wq = tid & 63, wrow = 16 * (tid >> 6) + (wq & 15), wk = 16 * (wq >> 4);
-    auto lstore = [&](int b, const Stage &r) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + 256 * i;
-            *reinterpret_cast<u32x4_t *>(&st[b].x[(c >> 3) * kPPitch + (c & 7) * 8]) = r.x[i];
-        }
-#pragma unroll
-        for (int gi = 0; gi < 2; ++gi) {
-            f16x8_t lo, hi;
-            i8x16_to_f16(r.w[gi], lo, hi);
-            uint16_t *d = &st[b].w[(64 * gi + wrow) * kPPitch + wk];
-            *reinterpret_cast<f16x8_t *>(d) = lo;
-            *reinterpret_cast<f16x8_t *>(d + 8) = hi;
-        }
-    };
-
-    // 32x32x16 fp16 MFMA: A lane l = W row (channel) l % 32, k 8 (l / 32)
-    // .. +7; B lane l = x row l % 32, the same k; C element e of lane l =
-    // channel 8 (e / 4) + 4 (l / 32) + e % 4, row l % 32
-    f32x16_t acc[2][2];  // [channel tile jt][row tile it], 32 x 32 each
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-        for (int it = 0; it < 2; ++it)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[jt][it][e] = 0.f;
-    const int l32 = lane & 31, h2 = lane >> 5;
-    auto compute = [&](int b) {
-        if (!active) return;
-#pragma unroll
-        for (int kk = 0; kk < 64; kk += 16) {
-            f16x8_t a[2], bx[2];
-#pragma unroll
-            for (int jt = 0; jt < 2; ++jt)
-                a[jt] = *reinterpret_cast<const f16x8_t *>(
-                    &st[b].w[(64 * wn + 32 * jt + l32) * kPPitch + kk + 8 * h2]);
-#pragma unroll
-            for (int it = 0; it < 2; ++it)
-                bx[it] = *reinterpret_cast<const f16x8_t *>(
-                    &st[b].x[(64 * wm + 32 * it + l32) * kPPitch + kk + 8 * h2]);
-#pragma unroll
-            for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-                for (int it = 0; it < 2; ++it)
-                    acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[jt], bx[it], acc[jt][it], 0, 0, 0);
-        }
-    };
-
-    // step s: registers R[s % 2], LDS buffer s % 2; the loop is unrolled by
-    // two so that every register stage is a fixed set of registers
-    // Loads are issued on every turn (past the last step they re-read it:
-    // in bounds, never stored), so that every path has the same loads in
-    // flight and the compiler waits only for the older stage.
-    Stage R0, R1;
-    const int last = steps - 1;
-    gload(0, R0);
-    gload(min(1, last), R1);
-    lstore(0, R0);
-    __syncthreads();
-    for (int s = 0; s < steps; s += 2) {
-        // even step s: R0 is free (stored at the previous turn)
-        gload(min(s + 2, last), R0);
-        compute(0);
-        if (s + 1 < steps) lstore(1, R1);
-        __syncthreads();
-        if (s + 1 >= steps) break;
-        // odd step s + 1: R1 is free
-        gload(min(s + 3, last), R1);
-        compute(1);
-        if (s + 2 < steps) lstore(0, R0);
-        __syncthreads();
-    }
-    if (!active) return;
-
-    // lane l of tile (jt, it): row m0 + 64 wm + 32 it + l % 32, channels from
-    // n0 + 64 wn + 32 jt
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int row = m0 + 64 * wm + 32 * it + l32;
-            if (row < M) w8p_store_tile(acc[jt][it], row, n0 + 64 * wn + 32 * jt, h2, scale, N, out);
-        }
-}
-
-// The large-tile form: block 256 rows x 256 channels, 8 waves as 2 x 4
-// (128 rows x 64 channels each: 4 x 2 tiles of 32x32x16 fp16 MFMA).  Both
-// operands of a 64-k step reach LDS by DMA (global_load_lds, 1 KB per wave
-// instruction): the 256 activation rows (32 KB) and the four 4 KB weight
-// tiles of the block's channel groups, copied as they lie.  The buffers
-// form a ring of three steps held in separate arrays, so that the compiler
-// can tell the slot being filled from the slot being read and does not wait
-// for the DMA before every LDS read; the loads of step s + 2 are issued
-// into the slot step s - 1 used, and one wait on the vector memory counter
-// before each barrier makes step s + 1's tiles complete.  An activation row
-// is 128 B; its 16-byte piece p sits in slot p ^ ((row / 2) % 8), so that
-// the 16 rows a quarter-wave reads cover all 64 banks.  The weights are
-// widened to fp16 from LDS.  Lane l of a 32-channel MFMA tile reads, from
-// 16-row weight tile 2 jt + (l % 32) / 16, row l % 16 and the 16-byte
-// pieces g' = l / 32 and l / 32 + 2 of the 64-k step (k 16 g' .. +15); MFMA
-// kk (4 per step) takes 8 of them: k = 32 (kk / 2) + 16 (l / 32) + 8 (kk %
-// 2) .. +7, and the activation (B) lanes read the same k.
-// Measured at M = 32768 on the 4B shapes: 12-19% faster than the same tile
-// with the weights loaded into registers and the activations staged through
-// registers (gate|up 1060-1086 against 933-965 TFLOP/s), bit-identical.
-constexpr int kPBM2 = 256;
-constexpr int kPBN2 = 256;
-// Rows from which the large-tile form is used: below two row blocks its
-// tile would be mostly padding.
-constexpr int kW8pLargeRows = 512;
-
 typedef __attribute__((address_space(3))) void lds_void_t;
+
+constexpr int kPBN = 256;                       // channels per block
+constexpr int kPScratch = 512;                  // epilogue scratch, floats per wave (2 KB)
+constexpr size_t kPPartWave = 2 * 16 * 64;      // floats of a wave's split partial per row tile
+
 // LDS index (halves) of the 16-byte piece `piece` of activation row `row`
 GDN_DEV int dswz(int row, int piece) { return row * 64 + ((piece ^ ((row >> 1) & 7)) << 3); }
 // wait until at most N vector memory operations of this wave are outstanding
 template <int N> GDN_DEV void wait_vm() { __builtin_amdgcn_s_waitcnt((N & 15) | 0x0F70 | ((N >> 4) << 14)); }
+// LDS DMA: lane l's 16 bytes at base + off[l] go to lds + 16 l (lds uniform).
+// Written as asm so that the compiler does not count it against the LDS reads
+// of the other ring slots (it would wait for every DMA before them); the
+// kernel's own wait_vm and barriers order it.  The compiler does not see that
+// the asm reads base in a vector memory operation: base must come from scalar
+// arithmetic, not straight from a readfirstlane (five wait states apart).
+GDN_DEV void dma16(const void *base, uint32_t off, uint32_t lds) {
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+                     : "memory");
+}
+GDN_DEV int scalar(int x) { return __builtin_amdgcn_readfirstlane(x); }
+GDN_DEV uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(const lds_void_t *)p; }
 // barrier that waits for this wave's LDS operations only (not for its DMA)
-GDN_DEV void lds_bar() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+GDN_DEV void lds_bar() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), as a builtin: the compiler drops its own waits for what it covers
+    __asm__ volatile("s_barrier" ::: "memory");
+}
+// silu(y) * up in fp32: the argument's product with log2(e) in two parts, so
+// that the exponential keeps its last bits; exp2 and the reciprocal are the
+// hardware's (1 ulp).
+GDN_DEV float silu_mul(float y, float up) {
+    const float t = y * -1.4426950408889634f;
+    const float r = fmaf(y, -1.4426950408889634f, -t);
+    const float e = __builtin_amdgcn_exp2f(t) * fmaf(r, 0.69314718f, 1.0f);
+    return y * __builtin_amdgcn_rcpf(1.0f + e) * up;
+}
 
-__global__ __launch_bounds__(512, 1) void w8p2_kernel(const uint16_t *__restrict__ X, int ldx,
-                                                      const int8_t *__restrict__ W, const float *__restrict__ scale,
-                                                      int M, int N, int K, W8Out out) {
-    __shared__ __align__(16) uint16_t xa[kPBM2 * 64];
-    __shared__ __align__(16) uint16_t xb[kPBM2 * 64];
-    __shared__ __align__(16) uint16_t xc[kPBM2 * 64];
-    __shared__ __align__(16) int8_t wa[4 * 4096];
-    __shared__ __align__(16) int8_t wb[4 * 4096];
-    __shared__ __align__(16) int8_t wc[4 * 4096];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int n0 = blockIdx.x * kPBN2, m0 = blockIdx.y * kPBM2;
-    const int steps = K / 64;
-    const int cg = n0 / 64 + wn;
-    const bool active = cg < N / 64;
-    const int l32 = lane & 31, h2 = lane >> 5;
-    const uint16_t *xsrc[4];
+// Epilogues of a wave's 32 IT rows x 64 channels (per row tile two 32x32
+// accumulator tiles; lane l holds, for q = 0..3, channels 32 jt + 8 q + 4 (l
+// / 32) .. +3 of row l % 32).  Each tile crosses the wave's scratch, so that
+// a row is stored as 128 contiguous bytes (SwiGLU: 64): stored from the
+// accumulators, every store instruction would touch 32 rows with 32 (16)
+// bytes each.  kW8tAdd is kW8Segments with one segment and a residual; its
+// loads run one row tile ahead of the stores (vector memory operations
+// complete in order, so a load behind a store would wait for it).
+enum W8tMode : int { kW8tSegments = 0, kW8tAdd = 1, kW8tSwiGLU = 2 };
+template <int IT, int MODE>
+GDN_DEV void w8t_epilogue(const f32x16_t (&acc)[IT][2], float *scratch, int row0, int nc,
+                          const float *__restrict__ scale, int M, int N, const W8Out &out) {
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h2 = lane >> 5;
+    if constexpr (MODE == kW8tSwiGLU) {
+        // 16-channel groups: 8 gate channels (q even), then their 8 up channels (q + 1)
+        f32x4_t sg[2][2], su[2][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = 32 * wave + 8 * i + (lane >> 3);
-        const int piece = (lane & 7) ^ ((row >> 1) & 7);
-        xsrc[i] = X + (size_t)min(m0 + row, M - 1) * ldx + piece * 8;
-    }
-    // weight DMA: wave w moves kilobytes 2w and 2w + 1 of the block's four
-    // 4 KB group tiles (group (2w + i) / 4, absent groups re-read group 0)
-    const int8_t *wsrc[2];
+        for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int kb = 2 * wave + i, g = kb >> 2;
-        const int gg = n0 / 64 + g < N / 64 ? n0 / 64 + g : 0;
-        wsrc[i] = W + (size_t)gg * steps * 4096 + (kb & 3) * 1024 + lane * 16;
-    }
-    auto dma = [&](int s, uint16_t *xbuf, int8_t *wbuf) {
+            for (int q2 = 0; q2 < 2; ++q2) {
+                const int n = nc + 32 * jt + 16 * q2 + 4 * h2;
+                sg[jt][q2] = *reinterpret_cast<const f32x4_t *>(scale + n);
+                su[jt][q2] = *reinterpret_cast<const f32x4_t *>(scale + n + 8);
+            }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds(xsrc[i] + s * 64, (lds_void_t *)(xbuf + (32 * wave + 8 * i) * 64), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            __builtin_amdgcn_global_load_lds(wsrc[i] + (size_t)s * 4096, (lds_void_t *)(wbuf + (2 * wave + i) * 1024), 16, 0, 0);
-    };
-    const int woff = wn * 4096 + (l32 >> 4) * 1024 + (16 * h2 + (l32 & 15)) * 16;
-    f32x16_t acc[2][4];
-#pragma unroll
-    for (int jt = 0; jt < 2; ++jt)
-#pragma unroll
-        for (int it = 0; it < 4; ++it)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[jt][it][e] = 0.f;
-    auto compute = [&](const uint16_t *buf, const int8_t *wbuf) {
-#pragma unroll
-        for (int pc = 0; pc < 2; ++pc) {
-            f16x8_t a[2][2];
+        for (int it = 0; it < IT; ++it) {
 #pragma unroll
             for (int jt = 0; jt < 2; ++jt)
-                i8x16_to_f16(*reinterpret_cast<const u32x4_t *>(wbuf + woff + jt * 2048 + pc * 512), a[jt][0], a[jt][1]);
 #pragma unroll
-            for (int k2 = 0; k2 < 2; ++k2) {
-                const int kk = 2 * pc + k2;
-                const int piece = 4 * (kk >> 1) + 2 * h2 + (kk & 1);
-                f16x8_t bx[4];
+                for (int q2 = 0; q2 < 2; ++q2) {
+                    float o[4];
 #pragma unroll
-                for (int it = 0; it < 4; ++it)
-                    bx[it] = *reinterpret_cast<const f16x8_t *>(&buf[dswz(128 * wm + 32 * it + l32, piece)]);
+                    for (int e = 0; e < 4; ++e)
+                        o[e] = silu_mul(acc[it][jt][8 * q2 + e] * sg[jt][q2][e],
+                                        acc[it][jt][8 * q2 + 4 + e] * su[jt][q2][e]);
+                    // a row's 32 outputs are four 16-byte pieces: piece 2 jt + q2, half h2
+                    const int slot = (2 * jt + q2) ^ ((l32 >> 2) & 3);
+                    *reinterpret_cast<uint2 *>(scratch + l32 * 16 + slot * 4 + 2 * h2) =
+                        make_uint2((uint32_t)f32_to_f16_rne(o[0]) | ((uint32_t)f32_to_f16_rne(o[1]) << 16),
+                                   (uint32_t)f32_to_f16_rne(o[2]) | ((uint32_t)f32_to_f16_rne(o[3]) << 16));
+                }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int rr = 16 * i + (lane >> 2), pc = lane & 3, row = row0 + 32 * it + rr;
+                const u32x4_t v = *reinterpret_cast<const u32x4_t *>(scratch + rr * 16 + ((pc ^ ((rr >> 2) & 3)) << 2));
+                if (row < M) *reinterpret_cast<u32x4_t *>(out.x16 + (size_t)row * (N / 2) + nc / 2 + 8 * pc) = v;
+            }
+        }
+    } else {
+        const int pc = lane & 7;  // the lane's four channels (of each 32) on the way out
+        f32x4_t sc[2];
+        float *dst[2];
+        int ld[2];
+        bool ok[2];  // channels past the last segment: padding
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt) {
+            const int n = nc + 32 * jt + 4 * pc;
+            sc[jt] = *reinterpret_cast<const f32x4_t *>(scale + n);
+            ok[jt] = n < out.seg[out.nseg - 1].n_end;
+            int nb = 0;
+            dst[jt] = out.seg[0].dst;
+            ld[jt] = out.seg[0].ld;
+            if constexpr (MODE == kW8tSegments) {
+#pragma unroll
+                for (int qq = 1; qq < kW8MaxSegs; ++qq)
+                    if (qq < out.nseg && n >= out.seg[qq - 1].n_end) {
+                        nb = out.seg[qq - 1].n_end;
+                        dst[jt] = out.seg[qq].dst;
+                        ld[jt] = out.seg[qq].ld;
+                    }
+            }
+            dst[jt] += n - nb;
+        }
+        // the residual of row tile it (rows past M and padding read an
+        // element in bounds, never stored); it may be in place: each element
+        // is read and written by one lane
+        f32x4_t res[2][8];
+        auto load_res = [&](int it) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int jt = j >> 2, row = min(row0 + 32 * it + 8 * (j & 3) + (lane >> 3), M - 1);
+                res[it & 1][j] = *reinterpret_cast<const f32x4_t *>(
+                    out.add_in + (size_t)row * out.add_ld + (ok[jt] ? nc + 32 * jt + 4 * pc : 0));
+            }
+        };
+        if constexpr (MODE == kW8tAdd) load_res(0);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            if constexpr (MODE == kW8tAdd)
+                if (it + 1 < IT) load_res(it + 1);
+#pragma unroll
+            for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    if ((l32 >> 4) == half)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            *reinterpret_cast<f32x4_t *>(scratch + (l32 & 15) * 32 + (((2 * q + h2) ^ (l32 & 7)) << 2)) =
+                                f32x4_t{acc[it][jt][4 * q], acc[it][jt][4 * q + 1], acc[it][jt][4 * q + 2],
+                                        acc[it][jt][4 * q + 3]};
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int rr = 8 * i + (lane >> 3), row = row0 + 32 * it + 16 * half + rr;
+                        f32x4_t y =
+                            *reinterpret_cast<const f32x4_t *>(scratch + rr * 32 + ((pc ^ (rr & 7)) << 2)) * sc[jt];
+                        if constexpr (MODE == kW8tAdd) y = res[it & 1][4 * jt + 2 * half + i] + y;
+                        // pinned ahead of the branch: a load that is waited for only inside it would
+                        // leave the compiler a wait for every DMA at the head of the main loop
+                        __asm__ volatile("" : "+v"(y));
+                        if (row < M && ok[jt]) *reinterpret_cast<f32x4_t *>(dst[jt] + (size_t)row * ld[jt]) = y;
+                    }
+                }
+        }
+    }
+}
+
+// The launch's work units: below `full`, unit u is one output tile over all
+// of K; from there, part (u - full) % S of the k-steps of tile full +
+// (u - full) / S, its sums going to `part` unscaled for w8t_reduce_kernel.
+// Blocks take units blockIdx, blockIdx + grid, ...; unit u runs on XCD u % 8
+// (blocks are handed out round robin and the grid is a multiple of 8).
+struct W8tPlan {
+    int tiles_m, tiles_n, full, S, units, grid;
+};
+// First k-step of part sp of S.
+GDN_DEV int w8t_part(int ksteps, int sp, int S) { return ksteps / S * sp + min(sp, ksteps % S); }
+// Tile index of a unit -> (row block, channel block).  Each XCD takes a
+// contiguous range of the whole tiles, four row blocks at a time, so that
+// the tiles its CUs work on at once share activation and weight tiles in
+// its L2.  S splits of a tile go to different XCDs, the same k-range of
+// neighbouring tiles to the same one.
+GDN_DEV void w8t_tile(const W8tPlan &p, int t, int &tm, int &tn) {
+    const int n = p.full / 8;
+    if (t < 8 * n) t = (t % 8) * n + t / 8;
+    const int per = 4 * p.tiles_n, gi = t / per, r = t - gi * per;
+    const int h = min(4, p.tiles_m - gi * 4);
+    tn = r / h;
+    tm = gi * 4 + r - tn * h;
+}
+
+// Block 64 IT rows x 256 channels (IT = 4, 2, 1), 8 waves as 2 x 4 (32 IT
+// rows x 64 channels each: IT x 2 tiles of 32x32x16 fp16 MFMA), persistent
+// over its units.  Both operands of a 64-k step reach LDS by DMA (1 KB per
+// wave instruction): the activation rows and the four 4 KB weight tiles of
+// the block's channel groups, copied as they lie, into a ring of three
+// steps; the DMA runs two steps ahead, across unit boundaries.  An
+// activation row is 128 B; its 16-byte piece p sits in slot p ^ ((row / 2) %
+// 8), so that the 16 rows a quarter-wave reads cover all 64 banks.  The
+// weights are widened to fp16 from LDS.  Lane l of a 32-channel MFMA tile
+// reads, from 16-row weight tile 2 jt + (l % 32) / 16, row l % 16 and the
+// 16-byte pieces g' = l / 32 and l / 32 + 2 of the 64-k step (k 16 g' ..
+// +15); MFMA kk (4 per step) takes 8 of them: k = 32 (kk / 2) + 16 (l / 32)
+// + 8 (kk % 2) .. +7, and the activation (B) lanes read the same k.
+//
+// What bounds it: at 256 rows the MFMA pipes under the chip's power limit
+// (zero operands run the 4B down matrix at 20000 rows in 616 us, random ones
+// in 845: the clock drops to 1.7 GHz), below that the latency of a step's
+// load half.  At 20000 rows against the kernel with one block per tile and a
+// store from the accumulators: gate|up 1842 -> 1616 us (fp32 out, 1168
+// TFLOP/s), in 1274 -> 1100, down 935 -> 753 (with the split last round; 845
+// without), out 451 -> 360; at 333 rows, down 105 -> 34 us, 30 of it the
+// split over k.  hipBLASLt's fp16 GEMM on the same shapes: 1515, 974, 822.
+//
+// Schedule, IT = 4: the waves of wave row 0 (one per SIMD) and of wave row 1
+// (the other one of each SIMD) run half a phase apart.  A phase is 32 k: first
+// its LDS reads, the weights' widening and the DMA requests ("load"), then
+// its 4 IT MFMAs ("multiply"), with a barrier after each half, so that on
+// every SIMD one wave multiplies while the other loads.  Ring safety, group
+// 0 half a phase ahead: the DMA of step s + 2 goes into the slot of step
+// s - 1, issued by group 0 in its load of (s, 0), one barrier after group
+// 1's load of (s - 1, 1) waited for its LDS reads; and every wave waits for
+// its own part of step s + 1 at the end of its load of (s, 1), which for
+// group 1 is one barrier before group 0's load of (s + 1, 0).
+// IT < 4: a phase's 4 IT MFMAs do not cover another wave's load half (0.83
+// us a step at IT = 2 that way, 0.69 this way), so each wave reads and widens
+// a phase ahead between its own MFMAs, with one barrier per step: the slot of
+// step s - 1 was last read before step s - 1's barrier, and the barrier of
+// step s follows every wave's wait for its part of step s + 1.  The ring is 4
+// (IT = 2) or 6 steps deep, what LDS holds.
+template <int IT, int MODE>
+__device__ __forceinline__ void w8t_body(const uint16_t *__restrict__ X, int ldx, const int8_t *__restrict__ W,
+                                         const float *__restrict__ scale, int M, int N, int K, const W8tPlan &plan,
+                                         float *__restrict__ part, const W8Out &out) {
+    constexpr int BM = 64 * IT;
+    constexpr int kRing = IT == 4 ? 3 : IT == 2 ? 4 : 6;  // steps of LDS (144, 128, 144 KB)
+    __shared__ __align__(16) uint16_t xs[kRing * BM * 64];
+    __shared__ __align__(16) int8_t ws[kRing * 4 * 4096];
+    __shared__ __align__(16) float scratch[8 * kPScratch];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 2, wn = wave & 3;  // waves w and w + 4 share a SIMD: one of each wave row
+    const int l32 = lane & 31, h2 = lane >> 5;
+    const int ksteps = K / 64;
+    // a unit's tile and k-steps
+    struct Unit {
+        int m0, n0, s0, s1;
+    };
+    auto unit_of = [&](int u) {
+        const bool split = u >= plan.full;
+        const int v = u - plan.full;
+        const int sp = split ? v % plan.S : 0;
+        int tm, tn;
+        w8t_tile(plan, split ? plan.full + v / plan.S : u, tm, tn);
+        return Unit{tm * BM, tn * kPBN, split ? w8t_part(ksteps, sp, plan.S) : 0,
+                    split ? w8t_part(ksteps, sp + 1, plan.S) : ksteps};
+    };
+
+    // ---- the DMA's cursor: the next step of unit du -------------------------
+    // activations: instruction i of wave w moves rows 8 (IT w + i) .. +7
+    // (rows past M read row M - 1, never stored); weights: wave w moves
+    // kilobytes 2w and 2w + 1 of the block's four 4 KB group tiles (group
+    // w / 2, absent groups re-read group 0)
+    int du = blockIdx.x, left;  // steps of unit du not requested yet, the next one included
+    const uint16_t *xnext;
+    const int8_t *wnext;
+    uint32_t xoff[IT];
+    const uint32_t loff = lane * 16;
+    auto dma_unit = [&]() {
+        const Unit t = unit_of(du);
+        left = scalar(t.s1 - t.s0);
+        const int wg = t.n0 / 64 + (wave >> 1) < N / 64 ? t.n0 / 64 + (wave >> 1) : 0;
+        const int r0 = min(t.m0 + 8 * IT * wave, M - 1);  // the wave's first row
+        xnext = X + (size_t)scalar(r0) * ldx + (size_t)scalar(t.s0) * 64;
+        wnext = W + ((size_t)scalar(wg) * ksteps + scalar(t.s0)) * 4096 + (2 * wave & 3) * 1024;
+        __asm__ volatile("s_nop 4" : "+s"(xnext), "+s"(wnext));  // see dma16
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int row = 8 * i + (lane >> 3);  // of the wave's 8 IT
+            const int piece = (lane & 7) ^ (((8 * IT * wave + row) >> 1) & 7);
+            xoff[i] = ((uint32_t)min(row, M - 1 - r0) * (uint32_t)ldx + piece * 8) * 2;
+        }
+    };
+    const uint32_t xl = lds_addr(xs) + (uint32_t)(IT * wave) * 1024, wl = lds_addr(ws) + (uint32_t)(2 * wave) * 1024;
+    auto dma_x = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < IT; ++i) dma16(xnext, xoff[i], xl + (uint32_t)(slot * (BM * 128) + i * 1024));
+    };
+    auto dma_w = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma16(wnext + i * 1024, loff, wl + (uint32_t)(slot * 16384 + i * 1024));
+    };
+    auto dma_advance = [&]() {
+        if (left > 1) {
+            --left;
+            xnext += 64;
+            wnext += 4096;
+        } else if (du + plan.grid < plan.units) {
+            du += plan.grid;
+            dma_unit();
+        }  // past the last unit its last step is read again (in bounds, never used)
+    };
+
+    f32x16_t acc[IT][2];
+    // MFMA operands of a phase (32 k, two 16-k MFMA groups)
+    struct Frags {
+        u32x4_t raw[2];
+        f16x8_t a[2][2], bx[2][IT];
+    };
+    const int woff = wn * 4096 + (l32 >> 4) * 1024 + (16 * h2 + (l32 & 15)) * 16;
+    auto lds_read = [&](Frags &f, int phase, int slot) {
+        const int8_t *wb = ws + slot * 16384 + woff + phase * 512;
+        const uint16_t *xb = xs + slot * (BM * 64);
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt) f.raw[jt] = *reinterpret_cast<const u32x4_t *>(wb + jt * 2048);
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int it = 0; it < IT; ++it)
+                f.bx[k2][it] = *reinterpret_cast<const f16x8_t *>(
+                    &xb[dswz(32 * IT * wm + 32 * it + l32, 4 * phase + 2 * h2 + k2)]);
+        __builtin_amdgcn_sched_barrier(0);  // every read requested before anything waits for one
+    };
+    auto widen = [&](Frags &f) {
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt) i8x16_to_f16(f.raw[jt], f.a[jt][0], f.a[jt][1]);
+    };
+    auto mult = [&](const Frags &f) {
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+                for (int it = 0; it < IT; ++it)
+                    acc[it][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[jt][k2], f.bx[k2][it], acc[it][jt], 0, 0, 0);
+    };
+    // IT = 4: the load half (reads already requested) and the multiply half of a phase
+    auto half_phases = [&](Frags &f) {
+        widen(f);
+        __builtin_amdgcn_sched_barrier(0);  // the widening belongs to the load half
+        lds_bar();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+        mult(f);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_bar();
+    };
+    // IT < 4: a phase's multiplies, the next phase's weights widened between them
+    auto mult_widen = [&](const Frags &f, Frags &next) {
+        mult(f);
+        widen(next);
+        // the first MFMAs cover the reads, then the widening goes between the rest
+        __builtin_amdgcn_sched_group_barrier(0x008, IT, 0);
+#pragma unroll
+        for (int i = 0; i < 3 * IT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, (40 + 3 * IT - 1) / (3 * IT), 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+    };
+
+    dma_unit();
+#pragma unroll
+    for (int i = 0; i < kRing - 1; ++i) {
+        dma_x(i);
+        dma_w(i);
+        dma_advance();
+    }
+    wait_vm<(kRing - 2) * (IT + 2)>();  // the first step landed
+    lds_bar();
+    Frags fa, fb;
+    int slot = 0, fill = kRing - 1;  // ring slots of the step multiplied and of the last step requested
+    if constexpr (IT == 4) {
+        if (wm == 1) lds_bar();  // half a phase behind
+    } else {
+        lds_read(fa, 0, 0);
+        widen(fa);
+    }
+    for (int u = blockIdx.x; u < plan.units; u += plan.grid) {
+        const Unit t = unit_of(u);
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+#pragma unroll
+            for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[it][jt][e] = 0.f;
+        for (int n = t.s1 - t.s0; n > 0; --n) {
+            const int nslot = slot == kRing - 1 ? 0 : slot + 1;
+            if constexpr (IT == 4) {
+                lds_read(fa, 0, slot);
+                dma_x(fill);
+                half_phases(fa);
+                lds_read(fa, 1, slot);
+                dma_w(fill);
+                dma_advance();
+                wait_vm<(kRing - 2) * (IT + 2)>();
+                half_phases(fa);
+            } else {
+                lds_read(fb, 1, slot);
+                dma_x(fill);
+                dma_w(fill);
+                dma_advance();
+                mult_widen(fa, fb);
+                wait_vm<(kRing - 2) * (IT + 2)>();
+                lds_bar();  // the step's reads are done, the next step's tiles are there
+                lds_read(fa, 0, nslot);
+                mult_widen(fb, fa);
+            }
+            fill = slot;
+            slot = nslot;
+        }
+        if (u >= plan.full) {
+            float *pp = part + ((size_t)(u - plan.full) * 8 + wave) * (IT * kPPartWave) + lane * 4;
+#pragma unroll
+            for (int it = 0; it < IT; ++it)
 #pragma unroll
                 for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-                    for (int it = 0; it < 4; ++it)
-                        acc[jt][it] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[jt][k2], bx[it], acc[jt][it], 0, 0, 0);
-            }
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<f32x4_t *>(pp + ((it * 2 + jt) * 4 + q) * 256) = f32x4_t{
+                            acc[it][jt][4 * q], acc[it][jt][4 * q + 1], acc[it][jt][4 * q + 2], acc[it][jt][4 * q + 3]};
+        } else if (t.n0 / 64 + wn < N / 64) {
+            w8t_epilogue<IT, MODE>(acc, scratch + wave * kPScratch, t.m0 + 32 * IT * wm, t.n0 + 64 * wn, scale, M, N,
+                                   out);
         }
-    };
-    const int last = steps - 1;
-    dma(0, xa, wa);
-    dma(min(1, last), xb, wb);
-    wait_vm<6>();  // step 0 landed
-    lds_bar();
-    // step s: its tiles in ring slot s % 3; the tiles of step s + 2 go into
-    // the slot step s - 1 used; step s + 1's tiles must land before the
-    // barrier that ends step s (after them come the 6 loads of step s + 2)
-#define W8P2_STEP(S, CX, CW, NX, NW)             \
-    dma(min((S) + 2, last), NX, NW);             \
-    compute(CX, CW);                             \
-    wait_vm<6>();                                \
-    lds_bar();                                   \
-    if ((S) + 1 >= steps) break;
-    for (int s = 0;; s += 3) {
-        W8P2_STEP(s, xa, wa, xc, wc)
-        W8P2_STEP(s + 1, xb, wb, xa, wa)
-        W8P2_STEP(s + 2, xc, wc, xb, wb)
     }
-#undef W8P2_STEP
-    wait_vm<0>();
-    if (!active) return;
+    if constexpr (IT == 4)
+        if (wm == 0) lds_bar();
+    wait_vm<0>();  // no DMA in flight into LDS the block gives back
+}
+
+template <int IT, int MODE>
+__global__ __launch_bounds__(512, 1) void w8t_kernel(const uint16_t *__restrict__ X, int ldx,
+                                                     const int8_t *__restrict__ W, const float *__restrict__ scale,
+                                                     int M, int N, int K, W8tPlan plan, float *__restrict__ part,
+                                                     W8Out out) {
+    w8t_body<IT, MODE>(X, ldx, W, scale, M, N, K, plan, part, out);
+}
+
+// Sums the S parts of every split tile in part order and runs the tile's
+// epilogue, with the multiplying kernel's wave and lane mapping: block
+// (split tile, row tile it of each wave).
+template <int IT, int MODE>
+__global__ __launch_bounds__(512) void w8t_reduce_kernel(const float *__restrict__ part,
+                                                         const float *__restrict__ scale, int M, int N,
+                                                         W8tPlan plan, W8Out out) {
+    __shared__ __align__(16) float scratch[8 * kPScratch];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave >> 2, wn = wave & 3, it = blockIdx.y;
+    int tm, tn;
+    w8t_tile(plan, plan.full + blockIdx.x, tm, tn);
+    const int nc = tn * kPBN + 64 * wn, row0 = tm * 64 * IT + 32 * (IT * wm + it);
+    if (nc >= N || row0 >= M) return;  // wave-uniform; no barriers below
+    const float *pp =
+        part + ((size_t)blockIdx.x * plan.S * 8 + wave) * (IT * kPPartWave) + it * kPPartWave + lane * 4;
+    f32x16_t acc[1][2];
 #pragma unroll
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            const int row = m0 + 128 * wm + 32 * it + l32;
-            if (row < M) w8p_store_tile(acc[jt][it], row, n0 + 64 * wn + 32 * jt, h2, scale, N, out);
-        }
+        for (int e = 0; e < 16; ++e) acc[0][jt][e] = 0.f;
+    for (int s = 0; s < plan.S; ++s) {
+        f32x4_t y[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            y[q] = *reinterpret_cast<const f32x4_t *>(pp + (size_t)s * 8 * (IT * kPPartWave) + q * 256);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[0][q >> 2][4 * (q & 3) + e] += y[q][e];
+    }
+    w8t_epilogue<1, MODE>(acc, scratch + wave * kPScratch, row0, nc, scale, M, N, out);
 }
 
 // ---- causal prefill attention ------------------------------------------------
@@ -558,26 +703,131 @@ __global__ __launch_bounds__(kApThreads) void attn_prefill_kernel(
 
 }  // namespace
 
-long long w8p_max_rows() { return 65535LL * kPBM2; }
+long long w8p_max_rows() { return 65535LL * 256; }
 
-hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int N, int K,
-                      const W8Out &out, hipStream_t st) {
+namespace {
+
+constexpr int kW8tBlocks = 256;              // one block per CU
+constexpr int kW8tMaxSplits = 8;
+constexpr int kW8tMinSteps = 4;              // k-steps of a split part at least
+constexpr int kW8tTailRows = 4096;           // rows from which only the last round's tiles are split
+constexpr size_t kW8tPartBytes = 384u << 20; // partial sums of one launch at most
+
+struct W8tChoice {
+    int it = 1;
+    W8tPlan plan{};
+    size_t part_bytes = 0;
+};
+
+W8tPlan w8t_plan(int M, int N, int it, int S, bool tail) {
+    W8tPlan p{};
+    p.tiles_m = (M + 64 * it - 1) / (64 * it);
+    p.tiles_n = (N + kPBN - 1) / kPBN;
+    const int tiles = p.tiles_m * p.tiles_n;
+    p.full = S == 1 ? tiles : tail ? tiles / kW8tBlocks * kW8tBlocks : 0;
+    p.S = S;
+    p.units = p.full + (tiles - p.full) * S;
+    p.grid = std::min(p.units, kW8tBlocks);
+    return p;
+}
+size_t w8t_part_bytes(const W8tPlan &p, int it) {
+    return (size_t)(p.units - p.full) * 8 * it * kPPartWave * sizeof(float);
+}
+// Modelled time (us) of a plan, from sweeps over the 4B matrices at 64 to
+// 20000 rows: a 64-k step of a block takes 1.05 / 0.68 / 0.54 us (IT = 4, 2,
+// 1) with few blocks on the chip and 1.5 / 0.92 / 0.65 us with all 256 (the
+// power limit lowers the clock), a tile's epilogue about IT us, a split
+// launch its second kernel and its partial sums written and read at about
+// 4.5 TB/s.  The model ranks the measured plans as they measured within 10%.
+double w8t_cost(const W8tPlan &p, int it, int ksteps) {
+    const int i = it == 4 ? 2 : it - 1;
+    const double few[3] = {0.54, 0.68, 1.05}, all[3] = {0.65, 0.92, 1.5};
+    const double load = (double)p.grid / kW8tBlocks, step = few[i] + (all[i] - few[i]) * load;
+    const int split_units = p.units - p.full;
+    const int rounds = (p.full + kW8tBlocks - 1) / kW8tBlocks;
+    double t = rounds * (ksteps * step + it);
+    if (split_units > 0) {
+        const int parts = (split_units + kW8tBlocks - 1) / kW8tBlocks;
+        t += parts * ((ksteps + p.S - 1) / p.S * step + it) + 4.0 + 2.0 * w8t_part_bytes(p, it) / 4.5e6;
+    }
+    return t;
+}
+// The row tile (64 IT) and the k-splits of M rows made of sequences of
+// `seq_rows` rows each, at most max_rows together.  The split decides the
+// order of a sum, so it is chosen without M (a sequence's result does not
+// depend on how many sequences it is batched with); the row tile does not
+// change a bit and is chosen for M.  Below kW8tTailRows every tile is split alike; from
+// there (where a launch holds one sequence) only the tiles left over after
+// the whole rounds of 256.
+W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, size_t part_limit) {
+    const int ksteps = K / 64;
+    const bool tail = seq_rows >= kW8tTailRows;
+    part_limit = std::min(part_limit, kW8tPartBytes);
+    const auto it_fits = [&](int it) { return (uint64_t)(8 * it) * ldx * 2 < (1ull << 32); };  // 32-bit row offsets
+    int S = 1;
+    double best = 1e30;
+    for (int s = 1; s <= kW8tMaxSplits && (s == 1 || ksteps / s >= kW8tMinSteps); ++s)
+        for (int it = 1; it <= 4; it *= 2) {
+            if (!it_fits(it)) continue;
+            // 256-row tiles bound the padded rows of every IT
+            const W8tPlan worst = w8t_plan(tail ? seq_rows : max_rows, N, tail ? it : 4, s, tail);
+            if (s > 1 && w8t_part_bytes(worst, tail ? it : 4) > part_limit) continue;
+            const double c = w8t_cost(w8t_plan(seq_rows, N, it, s, tail), it, ksteps);
+            if (c < best) {
+                best = c;
+                S = s;
+            }
+        }
+    W8tChoice r;
+    best = 1e30;
+    for (int it = 1; it <= 4; it *= 2) {
+        if (!it_fits(it)) continue;
+        const W8tPlan p = w8t_plan(M, N, it, S, tail);
+        const size_t pb = w8t_part_bytes(p, it);
+        const double c = w8t_cost(p, it, ksteps);
+        if (pb <= part_limit && c < best) {
+            best = c;
+            r = W8tChoice{it, p, pb};
+        }
+    }
+    return r;
+}
+
+template <int IT, int MODE>
+hipError_t w8t_run(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int N, int K,
+                   const W8tPlan &p, float *part, const W8Out &out, hipStream_t st) {
+    w8t_kernel<IT, MODE><<<p.grid, 512, 0, st>>>(x, ldx, W, scale, M, N, K, p, part, out);
+    const int split = p.tiles_m * p.tiles_n - p.full;
+    if (split > 0) w8t_reduce_kernel<IT, MODE><<<dim3(split, IT), 512, 0, st>>>(part, scale, M, N, p, out);
+    return hipGetLastError();
+}
+template <int MODE>
+hipError_t w8t_run_it(const W8tChoice &c, const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int N,
+                      int K, float *part, const W8Out &out, hipStream_t st) {
+    if (c.it == 4) return w8t_run<4, MODE>(x, ldx, W, scale, M, N, K, c.plan, part, out, st);
+    if (c.it == 2) return w8t_run<2, MODE>(x, ldx, W, scale, M, N, K, c.plan, part, out, st);
+    return w8t_run<1, MODE>(x, ldx, W, scale, M, N, K, c.plan, part, out, st);
+}
+
+}  // namespace
+
+size_t w8p_part_bytes(int M, int N, int K) { return w8t_choose(M, M, M, N, K, K, kW8tPartBytes).part_bytes; }
+size_t w8p_part_bytes_max() { return kW8tPartBytes; }
+
+hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
+                      int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st) {
     if (M <= 0) return hipSuccess;
-    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 ||
+    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 || M > w8p_max_rows() ||
+        seq_rows <= 0 || seq_rows > M || max_rows < M ||
+        (uint64_t)8 * ldx * 2 >= (1ull << 32) || (uintptr_t)part % 16 ||
         (out.mode != kW8Segments && out.mode != kW8SwiGLU) || (out.mode == kW8SwiGLU && (N % 16 || !out.x16)) ||
         (out.mode == kW8Segments && (out.nseg < 1 || out.nseg > kW8MaxSegs)) ||
         (out.add_in && (out.mode != kW8Segments || out.nseg != 1)))
         return hipErrorInvalidValue;
-    if (M >= kW8pLargeRows) {
-        const long long mb = (M + kPBM2 - 1) / kPBM2;
-        if (mb > 65535) return hipErrorInvalidValue;
-        w8p2_kernel<<<dim3((unsigned)((N + kPBN2 - 1) / kPBN2), (unsigned)mb), 512, 0, st>>>(x, ldx, W, scale, M, N,
-                                                                                           K, out);
-        return hipGetLastError();
-    }
-    const long long mb = (M + kPBM - 1) / kPBM;
-    w8p_kernel<<<dim3((unsigned)((N + kPBN - 1) / kPBN), (unsigned)mb), 256, 0, st>>>(x, ldx, W, scale, M, N, K, out);
-    return hipGetLastError();
+    const W8tChoice c = w8t_choose(M, seq_rows, max_rows, N, K, ldx, part ? part_bytes : 0);
+    if (out.mode == kW8SwiGLU) return w8t_run_it<kW8tSwiGLU>(c, x, ldx, W, scale, M, N, K, part, out, st);
+    if (out.add_in) return w8t_run_it<kW8tAdd>(c, x, ldx, W, scale, M, N, K, part, out, st);
+    return w8t_run_it<kW8tSegments>(c, x, ldx, W, scale, M, N, K, part, out, st);
 }
 
 hipError_t launch_attn_prefill(const uint16_t *q16, const uint16_t *Kc, const uint16_t *vT, const float *gate,

@@ -125,6 +125,53 @@ def test_w8a16_gemm_tiled_vs_oracle(L, M, N, K):
     assert not cnt.any()
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 2560, 9216),    # 64-row tiles, k split eight ways
+                                   (65, 2560, 2560),    # 40 k-steps: uneven parts
+                                   (129, 640, 4096),    # three channel blocks, the last with half its groups
+                                   (333, 2560, 9216), (700, 12352, 2560),
+                                   (1023, 2560, 4096),  # the last tile one row short
+                                   (4097, 1216, 1024),  # only the last round's tiles split
+                                   (5000, 18432, 512)])
+def test_w8a16_gemm_many_rows_workspaces(L, M, N, K):
+    """The many-row GEMM with the workspace the query asks for, with half of
+    it and with none: k-splits change only the order of the fp32 sums.  Bound:
+    each side within K * 2^-24 of the sum of the products' magnitudes (the
+    products are exact, every fp32 add rounds at most once at most that sum).
+    A call with M <= 16 before and after on the same uninitialised-past-its-own
+    workspace gives the same bits (its counters survive)."""
+    torch = torch_mod()
+    rs = np.random.RandomState(M + N + K)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(int(rs.randint(1 << 30)))
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    w = torch.randint(-127, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+    sc = torch.rand(N, generator=g, device="cuda") * 1e-2
+    wt = torch.empty_like(w)
+    assert L.kai_run_gdn_w8_tile_hip(P(w), P(wt), N, K, stream()) == 0
+    fn, need = L.kai_run_gdn_w8a16_gemm_tiled_hip, L.kai_gdn_w8a16_gemm_tiled_workspace_bytes
+    nb, nb8 = need(M, N, K), need(8, N, K)
+    ws = torch.full((max(nb, nb8, 256),), 0x7F, dtype=torch.uint8, device="cuda")
+    ws[:nb8] = 0
+
+    def small():
+        y = torch.empty(8, N, device="cuda")
+        assert fn(P(x), P(wt), P(sc), P(y), 8, N, K, P(ws), nb8, stream()) == 0
+        return y
+
+    y8 = small()
+    ref = x.double() @ w.double().t() * sc.double()
+    bound = (x.double().abs() @ w.double().abs().t() * sc.double()) * (K * 2.0 ** -24)
+    for use in (nb, nb // 2, 0):
+        y = torch.full((M, N), float("nan"), device="cuda")
+        assert fn(P(x), P(wt), P(sc), P(y), M, N, K, P(ws) if use else None, use, stream()) == 0
+        err = (y.double() - ref).abs()
+        assert bool((err <= bound).all()), (use, float((err / bound).max()))
+        y2 = torch.empty_like(y)
+        assert fn(P(x), P(wt), P(sc), P(y2), M, N, K, P(ws) if use else None, use, stream()) == 0
+        assert torch.equal(y, y2)
+    assert torch.equal(y8, small())
+
+
 def test_w8a16_gemm_tiled_rejects_bad_args(L):
     torch = torch_mod()
     t = empty((16 * 4096,), torch.float32)
