@@ -204,18 +204,28 @@ __global__ __launch_bounds__(256) void attn_prologue_kernel(
 // (s2 + s3)) and the per-element arithmetic is attn_prologue_kernel's; a
 // wave keeps its rows' loads in flight together (one row per 256-thread
 // block left every block waiting on one load), and the transposed V copy
-// takes 8 positions of a dim per 16-byte store.  Row t is position t of
-// sequence seq; V^T positions past T in the last group are written as 0.
+// takes 8 positions of a dim per 16-byte store.  Row t of sequence blockIdx.z
+// of the launch is position t of sequence seq0 + blockIdx.z; V^T positions
+// from T to Tv (read with weight 0) are written as 0.
 constexpr int kApRows = 8;
 __global__ __launch_bounds__(256) void attn_prologue_rows_kernel(
     const float *__restrict__ qg, const float *__restrict__ kx, const float *__restrict__ vx,
     const float *__restrict__ q_norm, const float *__restrict__ k_norm, uint16_t *__restrict__ q16,
-    uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc, int Hq, int Hkv, int Tmax, int T, int seq, float theta,
+    uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc, int Hq, int Hkv, int Tmax, int T, int seq0, float theta,
     float eps, uint16_t *__restrict__ vT, int Tv) {
     const int slot = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int seq = seq0 + (int)blockIdx.z;
+    {  // the sequence's rows of the launch's arrays
+        const size_t z = blockIdx.z;
+        qg += z * T * Hq * 512;
+        kx += z * T * Hkv * 256;
+        vx += z * T * Hkv * 256;
+        q16 += z * T * Hq * 256;
+        vT += z * Hkv * 256 * Tv;
+    }
     const int r0 = ((int)blockIdx.x * 4 + wave) * kApRows;
-    if (r0 >= T) return;  // the whole wave
-    const int nr = min(kApRows, T - r0);
+    if (r0 >= (slot >= Hq + Hkv ? Tv : T)) return;  // the whole wave
+    const int nr = min(kApRows, T - r0);            // <= 0: V^T padding
     if (slot >= Hq + Hkv) {  // value head: the cache, and the transposed copy
         const int kv = slot - Hq - Hkv;
         uint16_t v[kApRows][4];
@@ -230,7 +240,7 @@ __global__ __launch_bounds__(256) void attn_prologue_rows_kernel(
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
                     Vc[(((size_t)seq * Hkv + kv) * Tmax + r0 + j) * 256 + 64 * c + lane] = v[j][c];
-        if (vT) {
+        {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 uint4 w;
@@ -464,9 +474,10 @@ struct kai_gdn_hybrid {
     uint16_t *x16 = nullptr, *act16 = nullptr, *q16 = nullptr, *o16 = nullptr;
     float *gemm_part = nullptr, *attn_ws = nullptr;
     uint32_t *gemm_cnt = nullptr;  // zero between launches
-    // prefill buffers, allocated by the first prefill for max_context rows
+    // prefill buffers, allocated by the first prefill for `rows` positions
+    // (of one sequence or of several short ones)
     struct Prefill {
-        int rows = 0, tv = 0;   // capacity (positions) and the V^T row length
+        int rows = 0;
         float *part = nullptr;  // k-split partials of the GEMMs, w8p_part_bytes_max() bytes
         float *h = nullptr, *qkv = nullptr, *z = nullptr, *a = nullptr, *b = nullptr;
         float *g = nullptr, *beta = nullptr, *kx = nullptr, *vx = nullptr, *hist = nullptr;
@@ -842,14 +853,24 @@ hipError_t step(kai_gdn_hybrid *m, const int32_t *tokens, int32_t *next, float *
 
 // ---- prefill -------------------------------------------------------------------
 
+// Prompts that fit this many rows together run through a layer as one
+// group: at a few hundred rows a launch's time hardly depends on the rows
+// (four 200-token prompts of the 4B model: 42 ms one after another).
+constexpr int kPrefillGroupRows = 4096;
+// Longest prompt (chunks of 64) the chunked delta rule runs as one segment
+// whatever the batch; longer ones run one sequence per call, so that their
+// segments, and with them their roundings, do not depend on the batch.
+constexpr int kPrefillGroupChunks = 11;
+
 hipError_t prefill_alloc(kai_gdn_hybrid *m) {
     if (m->pf.rows) return hipSuccess;
     const kai_gdn_hybrid_config &c = m->cfg;
-    const size_t R = (size_t)c.max_context;
+    const size_t R = std::max((size_t)c.max_context,
+                              std::min((size_t)c.max_batch * c.max_context, (size_t)kPrefillGroupRows));
     const int H = c.hidden, C = m->conv_dim, V = m->value_dim, Hk = c.gdn_k_heads, Hv = c.gdn_v_heads,
               Hq = c.attn_q_heads, Hkv = c.attn_kv_heads;
     kai_gdn_hybrid::Prefill &p = m->pf;
-    p.tv = (int)((R + 63) / 64 * 64);
+    const size_t vt = (size_t)Hkv * 256 * (R + 64 * (size_t)c.max_batch);  // rows padded to 64 per sequence
     const size_t x16w = std::max({(size_t)H, (size_t)V, (size_t)Hq * 256});
     TRY(alloc_t(m, &p.h, R * H));
     TRY(alloc_t(m, &p.qkv, R * std::max((size_t)C, (size_t)Hq * 512)));
@@ -868,40 +889,58 @@ hipError_t prefill_alloc(kai_gdn_hybrid *m) {
     TRY(alloc_t(m, &p.v, R * V));
     TRY(alloc_t(m, &p.o, R * V));
     TRY(alloc_t(m, &p.q16, R * Hq * 256));
-    TRY(alloc_t(m, &p.vT, (size_t)Hkv * 256 * p.tv));
-    // V^T past a prefill's length is read (with weight 0): keep it finite
-    TRY(hipMemset(p.vT, 0, (size_t)Hkv * 256 * p.tv * sizeof(uint16_t)));
+    TRY(alloc_t(m, &p.vT, vt));
     TRY(alloc(m, reinterpret_cast<void **>(&p.part), w8p_part_bytes_max()));
     p.rows = (int)R;
     return hipDeviceSynchronize();
 }
 
-hipError_t w8p(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, int M, const W8Out &o, hipStream_t st) {
-    return launch_w8p(x, ldx, w.q, w.s, M, M, M, w.N, w.K, o, m->pf.part, w8p_part_bytes_max(), st);
+// The rows of a prefill launch: nseq sequences of T.
+struct Rows {
+    int nseq, T;
+    int total() const { return nseq * T; }
+};
+// Sequences of T rows that run as one group at most (whatever the batch).
+int group_limit(const kai_gdn_hybrid *m, int T) {
+    return std::max(1, std::min(m->cfg.max_batch, kPrefillGroupRows / T));
 }
-// A branch matrix: h[t] += x[t] W^T for the T rows, the residual add in the
+hipError_t w8p(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, Rows r, const W8Out &o, hipStream_t st) {
+    return launch_w8p(x, ldx, w.q, w.s, r.total(), r.T, group_limit(m, r.T) * r.T, w.N, w.K, o, m->pf.part,
+                      w8p_part_bytes_max(), st);
+}
+// A branch matrix: h[t] += x[t] W^T for the rows, the residual add in the
 // GEMM's epilogue (in place), so no branch array is written and read back.
-hipError_t w8p_residual(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, int M, float *h, int H,
+hipError_t w8p_residual(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, Rows r, float *h, int H,
                         hipStream_t st) {
     W8Out o = segments({{h, H, H}});
     o.add_in = h;
     o.add_ld = H;
-    return w8p(m, x, ldx, w, M, o, st);
+    return w8p(m, x, ldx, w, r, o, st);
 }
 
-// One sequence's prompt through every layer at once: T rows of sequence b.
-// Leaves its states (recurrent state, conv cache, K/V cache) where the
-// decode step reads them and the normalised last row in x16 row b.
-hipError_t prefill_seq(kai_gdn_hybrid *m, const int32_t *tokens, int b, int T, hipStream_t st) {
+// out[b] = x[(b + 1) T - 1]: the sequences' last rows (H fp16, H % 8 == 0)
+__global__ __launch_bounds__(256) void last_rows_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ out,
+                                                        int T, int H) {
+    const size_t b = blockIdx.x;
+    for (int i = threadIdx.x; i < H / 8; i += 256)
+        reinterpret_cast<uint4 *>(out + b * H)[i] = reinterpret_cast<const uint4 *>(x + ((b + 1) * T - 1) * H)[i];
+}
+
+// The prompts of sequences b0 .. b0 + r.nseq - 1 through every layer at once.
+// Leaves their states (recurrent state, conv cache, K/V cache) where the
+// decode step reads them and the normalised last rows in x16 rows b0 ...
+hipError_t prefill_group(kai_gdn_hybrid *m, const int32_t *tokens, int b0, Rows r, hipStream_t st) {
     const kai_gdn_hybrid_config &c = m->cfg;
     const int H = c.hidden, C = m->conv_dim, V = m->value_dim, Hk = c.gdn_k_heads, Hv = c.gdn_v_heads,
               Hq = c.attn_q_heads, Hkv = c.attn_kv_heads, I = c.inter;
+    const int T = r.T, R = r.total(), tv = pad64(T);
     kai_gdn_hybrid::Prefill &p = m->pf;
     TRY(mark(m, -1, st));
-    embed_kernel<<<T, 256, 0, st>>>(tokens, m->embed, p.h, H, c.vocab);
+    embed_kernel<<<R, 256, 0, st>>>(tokens, m->embed, p.h, H, c.vocab);
     TRY(hipGetLastError());
-    addnorm_kernel<<<T, 256, 0, st>>>(p.h, nullptr, m->layers[0].ln_in, p.x16, H, c.rms_eps);
+    addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, m->layers[0].ln_in, p.x16, H, c.rms_eps);
     TRY(hipGetLastError());
+    TRY(hipMemsetAsync(p.hist, 0, (size_t)3 * C * sizeof(float), st));
     TRY(mark(m, KAI_GDN_PHASE_OTHER, st));
     W8Out swiglu{};
     swiglu.mode = kW8SwiGLU;
@@ -909,51 +948,56 @@ hipError_t prefill_seq(kai_gdn_hybrid *m, const int32_t *tokens, int b, int T, h
     for (size_t l = 0; l < m->layers.size(); ++l) {
         Layer &L = m->layers[l];
         if (!L.attn) {
-            TRY(w8p(m, p.x16, H, L.in, T, segments({{p.qkv, C, C}, {p.z, V, C + V}, {p.b, Hv, C + V + Hv},
-                                                  {p.a, Hv, C + V + 2 * Hv}}), st));
+            TRY(w8p(m, p.x16, H, L.in, r, segments({{p.qkv, C, C}, {p.z, V, C + V}, {p.b, Hv, C + V + Hv},
+                                                     {p.a, Hv, C + V + 2 * Hv}}), st));
             TRY(mark(m, KAI_GDN_PHASE_GDN_PROJ, st));
             // the decode step's conv cache: the last four conv inputs
-            TRY(launch_conv_state_from_inputs(p.qkv, L.conv_state[0] + (size_t)b * C * 4, 1, T, C, st));
-            TRY(hipMemsetAsync(p.hist, 0, (size_t)3 * C * sizeof(float), st));
+            TRY(launch_conv_state_from_inputs(p.qkv, L.conv_state[0] + (size_t)b0 * C * 4, r.nseq, T, C, st));
             TRY(launch_conv_gating(p.qkv, L.conv_wt, p.hist, p.a, p.b, L.A_log, L.dt_bias, p.q, p.k, p.v, p.g,
-                                   p.beta, T, Hk, Hv, st));
-            float *S = L.S + (size_t)b * Hv * 128 * 128;
-            TRY(hipMemsetAsync(S, 0, (size_t)Hv * 128 * 128 * sizeof(float), st));
-            const int rc = kai_run_gdn_chunk_delta_rule_bf16_f32_hip(p.q, p.k, p.v, p.g, p.beta, p.o, S, 1, T, Hv,
-                                                                    Hk, 1.0f / sqrtf(128.0f), st);
-            if (rc) return (hipError_t)rc;
-            const size_t rows = (size_t)T * Hv;
+                                   p.beta, r.nseq, T, Hk, Hv, st));
+            const size_t s1 = (size_t)Hv * 128 * 128;
+            float *S = L.S + b0 * s1;
+            TRY(hipMemsetAsync(S, 0, r.nseq * s1 * sizeof(float), st));
+            const int together = (T + 63) / 64 <= kPrefillGroupChunks ? r.nseq : 1;
+            for (int i = 0; i < r.nseq; i += together) {
+                const size_t t0 = (size_t)i * T;
+                const int rc = kai_run_gdn_chunk_delta_rule_bf16_f32_hip(
+                    p.q + t0 * Hk * 128, p.k + t0 * Hk * 128, p.v + t0 * V, p.g + t0 * Hv, p.beta + t0 * Hv,
+                    p.o + t0 * V, S + i * s1, together, T, Hv, Hk, 1.0f / sqrtf(128.0f), st);
+                if (rc) return (hipError_t)rc;
+            }
+            const size_t rows = (size_t)R * Hv;
             prefill_gated_norm_kernel<<<(unsigned)((rows + 7) / 8), 256, 0, st>>>(p.o, p.z, L.norm_w, p.x16, rows,
                                                                                   c.rms_eps);
             TRY(hipGetLastError());
             TRY(mark(m, KAI_GDN_PHASE_GDN_CORE, st));
-            TRY(w8p_residual(m, p.x16, V, L.out, T, p.h, H, st));
+            TRY(w8p_residual(m, p.x16, V, L.out, r, p.h, H, st));
             TRY(mark(m, KAI_GDN_PHASE_GDN_OPROJ, st));
         } else {
             const int nq = Hq * 512, nkv = Hkv * 256;
-            TRY(w8p(m, p.x16, H, L.in, T, segments({{p.qkv, nq, nq}, {p.kx, nkv, nq + nkv}, {p.vx, nkv, nq + 2 * nkv}}),
+            TRY(w8p(m, p.x16, H, L.in, r, segments({{p.qkv, nq, nq}, {p.kx, nkv, nq + nkv}, {p.vx, nkv, nq + 2 * nkv}}),
                     st));
-            attn_prologue_rows_kernel<<<dim3((T + 4 * kApRows - 1) / (4 * kApRows), Hq + 2 * Hkv), 256, 0, st>>>(
-                p.qkv, p.kx, p.vx, L.q_norm, L.k_norm, p.q16, L.Kc, L.Vc, Hq, Hkv, m->tmax, T, b, c.rope_theta,
-                c.rms_eps, p.vT, p.tv);
+            attn_prologue_rows_kernel<<<dim3(tv / (4 * kApRows), Hq + 2 * Hkv, r.nseq), 256, 0, st>>>(
+                p.qkv, p.kx, p.vx, L.q_norm, L.k_norm, p.q16, L.Kc, L.Vc, Hq, Hkv, m->tmax, T, b0, c.rope_theta,
+                c.rms_eps, p.vT, tv);
             TRY(hipGetLastError());
-            const size_t kvrow = (size_t)b * Hkv * m->tmax * 256;
-            TRY(launch_attn_prefill(p.q16, L.Kc + kvrow, p.vT, p.qkv + 256, nq, p.x16, T, Hq, Hkv, m->tmax, p.tv,
+            const size_t kvrow = (size_t)b0 * Hkv * m->tmax * 256;
+            TRY(launch_attn_prefill(p.q16, L.Kc + kvrow, p.vT, p.qkv + 256, nq, p.x16, r.nseq, T, Hq, Hkv, m->tmax, tv,
                                     1.0f / 16.0f, st));
-            TRY(w8p_residual(m, p.x16, Hq * 256, L.out, T, p.h, H, st));
+            TRY(w8p_residual(m, p.x16, Hq * 256, L.out, r, p.h, H, st));
             TRY(mark(m, KAI_GDN_PHASE_ATTN, st));
         }
-        addnorm_kernel<<<T, 256, 0, st>>>(p.h, nullptr, L.ln_post, p.x16, H, c.rms_eps);
+        addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, L.ln_post, p.x16, H, c.rms_eps);
         TRY(hipGetLastError());
-        TRY(w8p(m, p.x16, H, L.gate_up, T, swiglu, st));
-        TRY(w8p_residual(m, p.act16, I, L.down, T, p.h, H, st));
+        TRY(w8p(m, p.x16, H, L.gate_up, r, swiglu, st));
+        TRY(w8p_residual(m, p.act16, I, L.down, r, p.h, H, st));
         const float *next_norm = l + 1 < m->layers.size() ? m->layers[l + 1].ln_in : m->final_norm;
-        addnorm_kernel<<<T, 256, 0, st>>>(p.h, nullptr, next_norm, p.x16, H, c.rms_eps);
+        addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, next_norm, p.x16, H, c.rms_eps);
         TRY(hipGetLastError());
         TRY(mark(m, KAI_GDN_PHASE_FFN, st));
     }
-    return hipMemcpyAsync(m->x16 + (size_t)b * H, p.x16 + (size_t)(T - 1) * H, (size_t)H * sizeof(uint16_t),
-                          hipMemcpyDeviceToDevice, st);
+    last_rows_kernel<<<r.nseq, 256, 0, st>>>(p.x16, m->x16 + (size_t)b0 * H, T, H);
+    return hipGetLastError();
 }
 
 hipError_t prefill(kai_gdn_hybrid *m, const int32_t *tokens, int batch, int T, int32_t *next, float *logits,
@@ -965,7 +1009,9 @@ hipError_t prefill(kai_gdn_hybrid *m, const int32_t *tokens, int batch, int T, i
     m->batch = batch;
     m->pos = 0;
     m->parity = 0;
-    for (int b = 0; b < batch; ++b) TRY(prefill_seq(m, tokens + (size_t)b * T, b, T, st));
+    const int group = group_limit(m, T);
+    for (int b = 0; b < batch; b += group)
+        TRY(prefill_group(m, tokens + (size_t)b * T, b, Rows{std::min(group, batch - b), T}, st));
     float *lg = logits ? logits : m->logits;
     TRY(mark(m, -1, st));
     TRY(gemm(m, m->x16, m->lm, segments({{lg, c.vocab, c.vocab}}), st));

@@ -98,12 +98,14 @@ hipError_t launch_prefill_seq(int narrow_state, const uint16_t *q, const uint16_
 // Gating prologue: conv output x [rows][(2 Hk + Hv) * 128] -> q, k (L2-normalised)
 // [rows][Hk][128], v [rows][Hv][128] (bf16 bit patterns or fp32), g, beta [rows][Hv].
 // The prefill's causal conv (K = 4, SiLU; tap-major weights conv_wt [4][C],
-// the three previous inputs in hist [3][C]) fused with the gating prologue
+// the three previous inputs in hist [3][C], the same for each of the nseq
+// sequences of T rows) fused with the gating prologue
 // into bf16 q, k, v and fp32 g, beta: bit for bit launch_conv_k4 followed by
 // launch_gating_prologue, without the conv's output array.
 hipError_t launch_conv_gating(const float *x, const float *conv_wt, const float *hist, const float *a,
                               const float *b, const float *A_log, const float *dt_bias, uint16_t *q, uint16_t *k,
-                              uint16_t *v, float *g, float *beta, int64_t T, int Hk, int Hv, hipStream_t st);
+                              uint16_t *v, float *g, float *beta, int nseq, int64_t T, int Hk, int Hv,
+                              hipStream_t st);
 hipError_t launch_gating_prologue(bool bf16, const float *x, const float *a, const float *b,
                                   const float *A_log, const float *dt_bias, void *q, void *k,
                                   void *v, float *g, float *beta, size_t rows, int Hk, int Hv,
@@ -203,14 +205,15 @@ size_t w8p_part_bytes(int M, int N, int K);
 size_t w8p_part_bytes_max();
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
                       int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st);
-// Causal attention of one sequence's T positions: q16 [T][Hq][256] fp16,
+// Causal attention of nseq sequences of T positions, every array with the
+// sequence as its first index: q16 [T][Hq][256] fp16,
 // Kc [Hkv][Tmax][256] tiled by 16 positions (kv_tiled_offset), vT
 // [Hkv][256][Tv] fp16 (V transposed; Tv % 64 == 0, Tv >= T, finite past T),
 // gate rows [T] of gate_row floats (head h's gate at h * 512 + d);
 // out16 [T][Hq][256] = fp16(softmax(q k^T * scaling) v * sigmoid(gate)).
 hipError_t launch_attn_prefill(const uint16_t *q16, const uint16_t *Kc, const uint16_t *vT, const float *gate,
-                               int gate_row, uint16_t *out16, int T, int Hq, int Hkv, int Tmax, int Tv,
-                               float scaling, hipStream_t st);
+                               int gate_row, uint16_t *out16, int nseq, int T, int Hq, int Hkv, int Tmax,
+                               int Tv, float scaling, hipStream_t st);
 // Attention decode over an fp16 KV cache (head_dim 256, Hq / Hkv <= 4):
 // out [B][Hq][256] fp32; `workspace` holds attn_workspace_bytes(B, Hq, L),
 // or attn_workspace_bytes_tiled(B, Hq, L) for a k_tiled launch (whose

@@ -170,12 +170,23 @@ __global__ __launch_bounds__(kThreads) void conv_gating_kernel(
     const float *__restrict__ x, const float *__restrict__ wt, const float *__restrict__ hist,
     const float *__restrict__ a, const float *__restrict__ b, const float *__restrict__ A_log,
     const float *__restrict__ dt_bias, OutT *__restrict__ q, OutT *__restrict__ k, OutT *__restrict__ v,
-    float *__restrict__ g, float *__restrict__ beta, int64_t T, int Hk, int Hv) {
+    float *__restrict__ g, float *__restrict__ beta, int64_t T, int Hk, int Hv, int rows) {
     const int tid = threadIdx.x, lane = tid & 15, grp = tid >> 4;
     const int H = 2 * Hk + Hv;
     const int64_t C = (int64_t)H * D;
     const int h = blockIdx.y * kGroups + grp;  // uniform over the group
-    const int64_t t0 = (int64_t)blockIdx.x * kConvRows, t1 = min(T, t0 + kConvRows);
+    const int64_t t0 = (int64_t)blockIdx.x * rows, t1 = min(T, t0 + rows);
+    {  // sequence blockIdx.z of the launch
+        const int64_t z0 = (int64_t)blockIdx.z * T;
+        x += z0 * C;
+        a += z0 * Hv;
+        b += z0 * Hv;
+        q += z0 * Hk * D;
+        k += z0 * Hk * D;
+        v += z0 * Hv * D;
+        g += z0 * Hv;
+        beta += z0 * Hv;
+    }
     if (h < H) {
         const int64_t c = (int64_t)h * D + 8 * lane;
         V8 w[4], hh[3];
@@ -301,13 +312,18 @@ hipError_t launch_gating_prologue(bool bf16, const float *x, const float *a, con
 
 hipError_t launch_conv_gating(const float *x, const float *conv_wt, const float *hist, const float *a,
                               const float *b, const float *A_log, const float *dt_bias, uint16_t *q, uint16_t *k,
-                              uint16_t *v, float *g, float *beta, int64_t T, int Hk, int Hv, hipStream_t st) {
-    if (T <= 0) return hipSuccess;
-    if (Hk <= 0 || Hv <= 0) return hipErrorInvalidValue;
+                              uint16_t *v, float *g, float *beta, int nseq, int64_t T, int Hk, int Hv,
+                              hipStream_t st) {
+    if (T <= 0 || nseq <= 0) return hipSuccess;
+    if (Hk <= 0 || Hv <= 0 || nseq > 65535) return hipErrorInvalidValue;
     const int H = 2 * Hk + Hv;
-    const dim3 grid((unsigned)((T + kConvRows - 1) / kConvRows), (unsigned)((H + kGroups - 1) / kGroups));
+    const int hb = (H + kGroups - 1) / kGroups;
+    // rows per block: kConvRows, halved while that leaves fewer than two blocks per CU
+    int rows = kConvRows;
+    while (rows > kConvU && (T + rows - 1) / rows * hb * nseq < 512) rows /= 2;
+    const dim3 grid((unsigned)((T + rows - 1) / rows), (unsigned)hb, (unsigned)nseq);
     conv_gating_kernel<uint16_t><<<grid, kThreads, 0, st>>>(x, conv_wt, hist, a, b, A_log, dt_bias, q, k, v, g, beta,
-                                                            T, Hk, Hv);
+                                                            T, Hk, Hv, rows);
     return hipGetLastError();
 }
 

@@ -526,6 +526,14 @@ __global__ __launch_bounds__(kApThreads) void attn_prefill_kernel(
     const int qb = (int)gridDim.x - 1 - (int)blockIdx.x;  // longest blocks first
     const int kv = blockIdx.y;
     const int rep = Hq / Hkv;
+    {  // sequence blockIdx.z of the launch
+        const size_t z = blockIdx.z;
+        q16 += z * T * Hq * kApD;
+        out16 += z * T * Hq * kApD;
+        gate += z * T * gate_row;
+        Kc += z * Hkv * Tmax * kApD;
+        vT += z * Hkv * kApD * Tv;
+    }
     const bool live = (wave & 3) < rep;                   // wave-uniform
     const int h = kv * rep + min(wave & 3, rep - 1);
     int qpos[kApT];
@@ -831,13 +839,13 @@ hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *
 }
 
 hipError_t launch_attn_prefill(const uint16_t *q16, const uint16_t *Kc, const uint16_t *vT, const float *gate,
-                               int gate_row, uint16_t *out16, int T, int Hq, int Hkv, int Tmax, int Tv,
-                               float scaling, hipStream_t st) {
-    if (T <= 0) return hipSuccess;
+                               int gate_row, uint16_t *out16, int nseq, int T, int Hq, int Hkv, int Tmax,
+                               int Tv, float scaling, hipStream_t st) {
+    if (T <= 0 || nseq <= 0) return hipSuccess;
     if (Hkv <= 0 || Hq % Hkv || Hq / Hkv > 4 || Tmax % 16 || Tmax < T || Tv % kApK || Tv < T)
         return hipErrorInvalidValue;
     const float sc_log2 = scaling * 1.4426950408889634f;
-    attn_prefill_kernel<<<dim3((unsigned)((T + kApQ - 1) / kApQ), (unsigned)Hkv), kApThreads, 0, st>>>(
+    attn_prefill_kernel<<<dim3((unsigned)((T + kApQ - 1) / kApQ), (unsigned)Hkv, (unsigned)nseq), kApThreads, 0, st>>>(
         q16, Kc, vT, gate, gate_row, out16, T, Hq, Hkv, Tmax, Tv, sc_log2);
     return hipGetLastError();
 }

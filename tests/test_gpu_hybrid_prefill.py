@@ -178,6 +178,28 @@ def test_prefill_rows_independent_and_replayable(hb, fixture):
         assert np.array_equal(l1[0].view(np.uint32), l2[b].view(np.uint32))
 
 
+@pytest.mark.parametrize("T,batch", [(1, 4), (70, 4),  # one group; GEMMs with k-splits
+                                     (704, 4),          # the longest prompt whose delta rule runs grouped
+                                     (705, 3),          # and the shortest one run per sequence
+                                     (1400, 4)])        # two sequences per group
+def test_prefill_groups_match_single_prompts(hb, T, batch):
+    """Prompts that run together give the bits each gives alone: the logits,
+    and (through the steps after it) the states and caches they leave."""
+    cfg = dict(layers=4, attn_every=2, hidden=1024, inter=2048, vocab=512, gdn_k_heads=8, gdn_v_heads=16,
+               attn_q_heads=8, attn_kv_heads=2, max_batch=4, max_context=1500, rope_theta=1.0e7, rms_eps=1e-6)
+    gm = hb.HybridModel(hb.config(**cfg), 11)
+    rs = np.random.RandomState(T)
+    tokens = rs.randint(0, cfg["vocab"], (batch, T)).astype(np.int32)
+    cont = rs.randint(0, cfg["vocab"], (2, batch)).astype(np.int32)
+    rows = [prefill(gm, tokens, cfg["vocab"])[1]] + [step(gm, t, cfg["vocab"])[1] for t in cont]
+    assert all(np.isfinite(r).all() for r in rows)
+    for b in range(batch):
+        alone = [prefill(gm, tokens[b:b + 1], cfg["vocab"])[1]] + [step(gm, t[b:b + 1], cfg["vocab"])[1] for t in cont]
+        for got, want in zip(alone, rows):
+            assert np.array_equal(got[0].view(np.uint32), want[b].view(np.uint32)), (T, b)
+    gm.close()
+
+
 def test_prefill_rejects_bad_arguments(hb, fixture):
     import orionsbelt_amd as ob
     torch = torch_mod()
