@@ -312,8 +312,10 @@ int kai_run_gdn_w8_quantize_hip(const float *W, int8_t *Wq, float *scale, int N,
  *   t < length, kv = h / (num_q_heads / num_kv_heads)
  * q [batch][num_q_heads][256] fp16 (after q_norm and RoPE), k_cache, v_cache
  * [batch][num_kv_heads][max_len][256] fp16, out fp32; softmax and sums in
- * fp32.  num_q_heads / num_kv_heads <= 4.  `workspace` holds at least
- * kai_gdn_attn_decode_workspace_bytes(batch, num_q_heads, length) bytes. */
+ * fp32.  num_q_heads / num_kv_heads <= 4.  `workspace` should hold
+ * kai_gdn_attn_decode_workspace_bytes(batch, num_q_heads, length) bytes; the
+ * least accepted is 1032 bytes per sequence, query head and 256 positions (a
+ * part counts whole), with which short contexts are split less and run slower. */
 size_t kai_gdn_attn_decode_workspace_bytes(int batch, int num_q_heads, int length);
 int kai_run_gdn_attn_decode_f16kv_hip(const uint16_t *q, const uint16_t *k_cache,
                                       const uint16_t *v_cache, float *out, int batch,

@@ -473,6 +473,7 @@ struct kai_gdn_hybrid {
     uint32_t *arg_cnt = nullptr;   // [max_batch], zero between launches
     uint16_t *x16 = nullptr, *act16 = nullptr, *q16 = nullptr, *o16 = nullptr;
     float *gemm_part = nullptr, *attn_ws = nullptr;
+    size_t attn_ws_bytes = 0;
     uint32_t *gemm_cnt = nullptr;  // zero between launches
     // prefill buffers, allocated by the first prefill for `rows` positions
     // (of one sequence or of several short ones)
@@ -771,7 +772,8 @@ hipError_t build(kai_gdn_hybrid *m, uint64_t seed) {
         TRY(alloc_t(m, &m->gemm_part, part));
         TRY(alloc_t(m, &m->gemm_cnt, groups));
         TRY(hipMemset(m->gemm_cnt, 0, groups * sizeof(uint32_t)));
-        TRY(alloc(m, reinterpret_cast<void **>(&m->attn_ws), attn_workspace_bytes_tiled(Bm, Hq, c.max_context)));
+        m->attn_ws_bytes = attn_workspace_bytes_tiled(Bm, Hq, c.max_context);
+        TRY(alloc(m, reinterpret_cast<void **>(&m->attn_ws), m->attn_ws_bytes));
         return hipDeviceSynchronize();
     };
     const hipError_t e = run();
@@ -807,7 +809,7 @@ hipError_t attn_mixer(kai_gdn_hybrid *m, Layer &L, hipStream_t st) {
     TRY(hipGetLastError());
     // o * sigmoid(gate) -> fp16 in the span combine; gate = dims 256..511 of each qg head
     TRY(launch_attn_decode(m->q16, L.Kc, L.Vc, nullptr, B, Hq, Hkv, m->tmax, m->pos + 1, 1.0f / 16.0f,
-                           m->attn_ws, st, m->qg + 256, 512, m->o16, /*k_tiled=*/true));
+                           m->attn_ws, m->attn_ws_bytes, st, m->qg + 256, 512, m->o16, /*k_tiled=*/true));
     TRY(gemm_addnorm(m, m->o16, L.out, m->mix, L.ln_post, st));
     return mark(m, KAI_GDN_PHASE_ATTN, st);
 }

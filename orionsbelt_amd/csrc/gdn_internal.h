@@ -215,19 +215,21 @@ hipError_t launch_attn_prefill(const uint16_t *q16, const uint16_t *Kc, const ui
                                int gate_row, uint16_t *out16, int nseq, int T, int Hq, int Hkv, int Tmax,
                                int Tv, float scaling, hipStream_t st);
 // Attention decode over an fp16 KV cache (head_dim 256, Hq / Hkv <= 4):
-// out [B][Hq][256] fp32; `workspace` holds attn_workspace_bytes(B, Hq, L),
-// or attn_workspace_bytes_tiled(B, Hq, L) for a k_tiled launch (whose
-// spans shrink to as few as 64 positions when the grid is small).
+// out [B][Hq][256] fp32.  `workspace` holds one partial per span: with
+// attn_workspace_bytes(B, Hq, L) (attn_workspace_bytes_tiled for any batch and
+// length up to these) the spans are as short as the grid wants, down to 64
+// positions; with less, at least attn_workspace_bytes_min, they are longer.
 // With `gate` (non-null), the output is instead out16 [B][Hq][256] fp16 =
 // fp16(o * sigmoid(gate[(b * Hq + h) * gate_stride + d])).
 // k_tiled: K is stored tiled by 16 positions (Tmax % 16 == 0), element
 // (t, d) of a (sequence, kv head) at kv_tiled_offset(t, d); V stays
 // row-major.
 size_t attn_workspace_bytes(int B, int Hq, int L);
-size_t attn_workspace_bytes_tiled(int B, int Hq, int L);  // the k_tiled launches' (shorter spans allowed)
+size_t attn_workspace_bytes_min(int B, int Hq, int L);
+size_t attn_workspace_bytes_tiled(int B, int Hq, int L);
 hipError_t launch_attn_decode(const uint16_t *q, const uint16_t *Kc, const uint16_t *Vc, float *out,
                               int B, int Hq, int Hkv, int Tmax, int L, float scaling, float *workspace,
-                              hipStream_t st, const float *gate = nullptr, int gate_stride = 0,
+                              size_t workspace_bytes, hipStream_t st, const float *gate = nullptr, int gate_stride = 0,
                               uint16_t *out16 = nullptr, bool k_tiled = false);
 // Offset (in halfs, from the row of position 0) of K[t][d] in the tiled
 // layout: group t / 16 holds 8 x 512 halfs; chunk j (dims 32 j .. 32 j + 31)

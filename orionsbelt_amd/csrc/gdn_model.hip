@@ -18,6 +18,8 @@
 // split k across blocks, into a partial-sum workspace that a second kernel
 // reduces in a fixed order (deterministic).  The layer is HBM-bound on the
 // weight bytes at decode sizes; the activations are L2-resident.
+#include <algorithm>
+
 #include "gdn_common.h"
 #include "gdn_internal.h"
 
@@ -740,9 +742,9 @@ hipError_t launch_w8f(const uint16_t *x, const int8_t *W, const float *scale, in
 // head h of sequence b, with kv = h / (Hq / Hkv) (repeat_kv),
 //   o[b][h] = softmax_t(scaling * q[b][h] . K[b][kv][t]) . V[b][kv][t],  t < L
 // q [B][Hq][256] fp16, K, V [B][Hkv][Tmax][256] fp16, fp32 softmax and sums.
-// Split over the sequence: block (span, kv, b) takes positions [256 span,
-// 256 span + 256) and every query head of kv; wave w takes 64 of them in
-// groups of 16.  Scores on fp16 MFMA 16x16x32 (A = 16 key rows, B = the
+// Split over the sequence: block (span, kv, b) takes 64 G consecutive
+// positions (attn_groups) and every query head of kv; wave w takes 16 G of
+// them in groups of 16.  Scores on fp16 MFMA 16x16x32 (A = 16 key rows, B = the
 // group's query heads as columns); online softmax per head in exp2; P.V on
 // the VALU, lane l holding dims 4l .. 4l+3 of every head's output.  The
 // block's four waves merge through LDS into one partial (max, sum, o) per
@@ -754,13 +756,14 @@ hipError_t launch_w8f(const uint16_t *x, const int8_t *W, const float *scale, in
 // ---------------------------------------------------------------------------
 namespace {
 
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 constexpr int kAttD = 256;
-constexpr int kAttSpan = 256;   // positions per block
+constexpr int kAttSpan = 256;   // positions per partial of the smallest workspace
 constexpr int kAttRepMax = 4;   // query heads per kv head handled (Hq / Hkv <= 4)
 constexpr int kAttPart = kAttD + 2;
 
 template <bool KTILED>
-__global__ __launch_bounds__(256) void attn_decode_kernel(const uint16_t *__restrict__ q,
+__global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__restrict__ q,
                                                           const uint16_t *__restrict__ Kc,
                                                           const uint16_t *__restrict__ Vc,
                                                           float *__restrict__ part, int Hq, int Hkv,
@@ -805,10 +808,12 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const uint16_t *__rest
             for (int j = 0; j < 8; ++j)
                 kb[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(kp + 512 * j));
         } else {
+            // cached loads: a row's 64-byte pieces of two loads share a 128-byte
+            // line (non-temporal, 8 x 12289 positions take 88 us instead of 78;
+            // V's whole 512-byte rows are faster non-temporal, 78 against 85)
             const uint16_t *kp = Kc + (kvrow + min(t0 + r, L - 1)) * kAttD + 8 * g;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                kb[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(kp + 32 * j));
+            for (int j = 0; j < 8; ++j) kb[j] = *reinterpret_cast<const u32x4_t *>(kp + 32 * j);
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i)
@@ -843,6 +848,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const uint16_t *__rest
         ps += __shfl_xor(ps, 32);
         const float alpha = __builtin_amdgcn_exp2f(mrow - mnew);  // 0 on the first group
         // every lane: the running state of each head from lane h
+        float a[kAttRepMax];
 #pragma unroll
         for (int h = 0; h < kAttRepMax; ++h) {
             if (h >= rep) break;
@@ -851,26 +857,33 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const uint16_t *__rest
             const float ps_h = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ps), h));
             m[h] = mn_h;
             l[h] = l[h] * a_h + ps_h;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[h][i] *= a_h;
+            a[h] = a_h;
         }
         // P.V: position t0 + 4gg + e, head h: p in lane 16 gg + h, element e
-        // (p = 0 for positions past L)
+        // (p = 0 for positions past L), summed over the group from zero, then
+        // added to the running output: the rounding of a span's sum then
+        // grows with 16 + its groups, not with its positions
+        float pv[kAttRepMax][4];
 #pragma unroll
         for (int gg = 0; gg < 4; ++gg)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const u32x2_t vv = vb[4 * gg + e];
-                const float v[4] = {f16_to_f32((uint16_t)(vv[0] & 0xFFFFu)), f16_to_f32((uint16_t)(vv[0] >> 16)),
-                                    f16_to_f32((uint16_t)(vv[1] & 0xFFFFu)), f16_to_f32((uint16_t)(vv[1] >> 16))};
+                const f16x4_t v = __builtin_bit_cast(f16x4_t, vb[4 * gg + e]);
 #pragma unroll
                 for (int h = 0; h < kAttRepMax; ++h) {
                     if (h >= rep) break;
                     const float ph = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p[e]), 16 * gg + h));
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) o[h][i] += ph * v[i];
+                    for (int i = 0; i < 4; ++i) pv[h][i] = gg == 0 && e == 0 ? ph * (float)v[i] : fmaf(ph, (float)v[i], pv[h][i]);
                 }
+                __builtin_amdgcn_sched_barrier(0);  // one position's V widened at a time
             }
+#pragma unroll
+        for (int h = 0; h < kAttRepMax; ++h) {
+            if (h >= rep) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[h][i] = fmaf(o[h][i], a[h], pv[h][i]);
+        }
     };
     if (t_begin < t_end) load_group(t_begin, kbuf[0], vbuf[0]);
     for (int t0 = t_begin; t0 < t_end; t0 += 32) {  // uniform over the wave
@@ -971,27 +984,36 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
 
 }  // namespace
 
-size_t attn_workspace_bytes(int B, int Hq, int L) {
-    const int nspan = (L + kAttSpan - 1) / kAttSpan;
-    return (size_t)B * Hq * nspan * kAttPart * sizeof(float);
-}
-
-// Groups of 16 positions per wave.  256-position spans (G = 4) for a
-// row-major K cache.  For a tiled-K cache the span is sized for a block
-// count: a grid of fewer than 2048 blocks of 256 positions fills 512 slots
-// (2 per CU on 256 CUs) in one round -- at B = 1 and 32K, 129 x 4 = 516
-// blocks of 256 positions would leave 4 blocks for a second round that
+namespace {
+// Groups of 16 positions per wave: the span (64 positions per group) is sized
+// for a block count.  A grid of fewer than 2048 blocks of 256 positions fills
+// 512 slots (2 per CU on 256 CUs) in one round -- at B = 1 and 32K, 129 x 4 =
+// 516 blocks of 256 positions would leave 4 blocks for a second round that
 // doubles the kernel's time -- and a larger grid is cut into about 2048
 // blocks: at B = 16 and 32K, spans of 16 groups (2112 blocks) took 356.5
-// against 381.4 us per layer with 4 groups (8256 blocks), decode and
-// combine, with 8 to 24 groups all within 364 us (longer spans read the
-// KV stream faster and leave fewer partials to combine).
-int attn_groups(int B, int Hkv, int L, bool k_tiled) {
-    const long blocks256 = (long)B * Hkv * ((L + kAttSpan - 1) / kAttSpan);
-    if (!k_tiled) return 4;
-    const int target = blocks256 >= 2048 ? 2048 : 512;
-    const int per_kv = max(1, target / (B * Hkv));
-    return max(1, (L + 64 * per_kv - 1) / (64 * per_kv));
+// against 381.4 us per layer with 4 groups (8256 blocks), decode and combine,
+// with 8 to 24 groups all within 364 us (longer spans read the KV stream
+// faster and leave fewer partials to combine).  Row-major caches, against
+// spans of 256 positions always: B = 8 at 12289 88 -> 78 us, B = 16 at 32K
+// 405 -> 364, B = 4 at 4096 23.2 -> 19.8, B = 1 at 2000 20.4 -> 9.6.
+int attn_groups(int B, int Hkv, int L) {
+    const long long pairs = (long long)B * Hkv, blocks256 = pairs * ((L + kAttSpan - 1LL) / kAttSpan);
+    const long long target = blocks256 >= 2048 ? 2048 : 512, per_kv = std::max(1LL, target / pairs);
+    return (int)((L + 64 * per_kv - 1) / (64 * per_kv));
+}
+size_t span_bytes(int B, int Hq, int nspan) { return (size_t)B * Hq * nspan * kAttPart * sizeof(float); }
+}  // namespace
+
+size_t attn_workspace_bytes_min(int B, int Hq, int L) { return span_bytes(B, Hq, (L + kAttSpan - 1) / kAttSpan); }
+
+size_t attn_workspace_bytes(int B, int Hq, int L) {
+    int nspan = (L + kAttSpan - 1) / kAttSpan;
+    for (int rep = 1; rep <= kAttRepMax; ++rep)
+        if (Hq % rep == 0) {
+            const int G = attn_groups(B, Hq / rep, L);
+            nspan = max(nspan, (int)((L + 64LL * G - 1) / (64LL * G)));
+        }
+    return span_bytes(B, Hq, nspan);
 }
 
 size_t attn_workspace_bytes_tiled(int B, int Hq, int L) {
@@ -1001,10 +1023,15 @@ size_t attn_workspace_bytes_tiled(int B, int Hq, int L) {
 
 hipError_t launch_attn_decode(const uint16_t *q, const uint16_t *Kc, const uint16_t *Vc, float *out,
                               int B, int Hq, int Hkv, int Tmax, int L, float scaling, float *workspace,
-                              hipStream_t st, const float *gate, int gate_stride, uint16_t *out16, bool k_tiled) {
+                              size_t workspace_bytes, hipStream_t st, const float *gate, int gate_stride,
+                              uint16_t *out16, bool k_tiled) {
     if (B == 0) return hipSuccess;
     if (k_tiled && Tmax % 16 != 0) return hipErrorInvalidValue;
-    const int G = attn_groups(B, Hkv, L, k_tiled);
+    // no more spans than the workspace holds
+    const size_t fit = workspace_bytes / span_bytes(B, Hq, 1);
+    if (fit == 0) return hipErrorInvalidValue;
+    const int cap = (int)std::min<size_t>(fit, 1u << 24);
+    const int G = max(attn_groups(B, Hkv, L), (int)((L + 64LL * cap - 1) / (64LL * cap)));
     const int nspan = (L + 64 * G - 1) / (64 * G);
     const float sc_log2 = scaling * 1.4426950408889634f;
     if (k_tiled)

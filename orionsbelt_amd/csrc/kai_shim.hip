@@ -885,11 +885,11 @@ extern "C" int kai_run_gdn_attn_decode_f16kv_hip(const uint16_t *q, const uint16
     if (!aligned(q, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(out, 16) ||
         !aligned(workspace, 16))
         return (int)hipErrorInvalidValue;
-    if (workspace_bytes < gdn::attn_workspace_bytes(batch, num_q_heads, length))
+    if (workspace_bytes < gdn::attn_workspace_bytes_min(batch, num_q_heads, length))
         return (int)hipErrorInvalidValue;
     return (int)gdn::launch_attn_decode(q, k_cache, v_cache, out, batch, num_q_heads, num_kv_heads,
                                         max_len, length, scaling, static_cast<float *>(workspace),
-                                        (hipStream_t)stream);
+                                        workspace_bytes, (hipStream_t)stream);
 }
 
 // ===========================================================================

@@ -263,6 +263,40 @@ def test_attn_decode_peaked_and_long(L):
         assert torch.allclose(out[0, h], v[0, kv, hot[kv]].float(), rtol=1e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,length", [(1, 4, 1, 17), (3, 16, 4, 63), (2, 8, 8, 65), (1, 16, 4, 257),
+                                             (5, 6, 2, 1000), (1, 16, 4, 4097),
+                                             (64, 16, 4, 2100),   # more than 2048 blocks of 256 positions
+                                             (130, 16, 4, 70)])   # more (sequence, kv head) pairs than blocks wanted
+def test_attn_decode_span_rule(L, B, Hq, Hkv, length):
+    """Spans sized by the grid (the queried workspace) and the longest spans
+    (the least workspace accepted), against 64-bit attention.  Bound per
+    output: a score is a sum of 256 exact products (error at most 260 * 2^-24
+    of their magnitudes), p's relative error at most twice the worst score's
+    plus one rounding per sum of `length` terms and its rescalings."""
+    torch = torch_mod()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(length)
+    cap, scal = length + 3, 1.0 / 16
+    q = torch.randn(B, Hq, 256, generator=g, device="cuda").half()
+    k, v = (torch.randn(B, Hkv, cap, 256, generator=g, device="cuda").half() for _ in range(2))
+    k[:, :, length:] = float("nan")          # positions past the length are never used
+    v[:, :, length:] = float("nan")
+    qd, kd, vd = q.double().reshape(B, Hkv, Hq // Hkv, 256), k.double()[:, :, :length], v.double()[:, :, :length]
+    p = torch.softmax(qd @ kd.transpose(2, 3).contiguous() * scal, -1)
+    ref = (p @ vd).reshape(B, Hq, 256)
+    es = (qd.abs() @ kd.abs().transpose(2, 3).contiguous()).max() * scal * 260 * 2.0 ** -24
+    bound = (p @ vd.abs()).reshape(B, Hq, 256) * (2 * es + (2 * length + 64) * 2.0 ** -24)
+    least = 1032 * B * Hq * ((length + 255) // 256)
+    for nb in (L.kai_gdn_attn_decode_workspace_bytes(B, Hq, length), least):
+        ws = torch.full((nb,), 0x7F, dtype=torch.uint8, device="cuda")
+        out = torch.full((B, Hq, 256), float("nan"), device="cuda")
+        assert L.kai_run_gdn_attn_decode_f16kv_hip(P(q), P(k), P(v), P(out), B, Hq, Hkv, cap, length, scal, P(ws), nb,
+                                                   stream()) == 0
+        assert bool(((out.double() - ref).abs() <= bound).all()), nb
+        assert L.kai_run_gdn_attn_decode_f16kv_hip(P(q), P(k), P(v), P(out), B, Hq, Hkv, cap, length, scal, P(ws),
+                                                   least - 4, stream()) != 0
+
+
 def test_attn_decode_rejects_bad_args(L):
     torch = torch_mod()
     t = empty((1 << 16,), torch.float32)
