@@ -251,3 +251,26 @@ def test_prologue_prefill_epilogue_chain(L):
     ry = orc.gated_rmsnorm_f32(ro.reshape(T * Hv, 128), bf16_to_f32(z), bf16_to_f32(w), 1e-6)
     mx, l2 = rel_errors(bf16_to_f32(y), ry)
     assert mx <= 3e-2 and l2 <= 1.5e-2, (mx, l2)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("Hk,Hv", [(16, 32), (3, 9)])
+def test_few_rows_match_many_rows(L, bf16, Hk, Hv):
+    """A row's bits do not depend on how many rows the call has: calls on
+    either side of the launch-shape rules (512 tokens in the prologue, 512
+    blocks of 64 fp32 or 128 bf16 rows in the norm) against one large call."""
+    rows = 700
+    x, a, b, A_log, dt = prologue_inputs(9, rows, Hk, Hv)
+    big = gpu_prologue(L, x, a, b, A_log, dt, rows, Hk, Hv, bf16)
+    for n in (1, 511, 512):
+        few = gpu_prologue(L, x[:n], a[:n], b[:n], A_log, dt, n, Hk, Hv, bf16)
+        for got, want in zip(few, big):
+            assert np.array_equal(got, want.reshape(rows, -1)[:n].reshape(got.shape)), n
+    rs = np.random.RandomState(10)
+    lim = 512 * (128 if bf16 else 64)
+    o, z, w = (rs.randn(*sh).astype(np.float32) for sh in ((lim + 5, 128), (lim + 5, 128), (128,)))
+    if bf16:
+        o, z, w = (orc.f32_to_bf16_bits(t) for t in (o, z, w))
+    big = gpu_rmsnorm(L, o, z, w, 1e-6, bf16)
+    for n in (1, 33, lim - 1, lim):
+        assert np.array_equal(gpu_rmsnorm(L, o[:n], z[:n], w, 1e-6, bf16), big[:n]), n
