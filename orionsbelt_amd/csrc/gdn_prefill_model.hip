@@ -232,8 +232,8 @@ GDN_DEV void w8t_tile(const W8tPlan &p, int t, int &tm, int &tn) {
 // load half.  At 20000 rows against the kernel with one block per tile and a
 // store from the accumulators: gate|up 1842 -> 1616 us (fp32 out, 1168
 // TFLOP/s), in 1274 -> 1100, down 935 -> 753 (with the split last round; 845
-// without), out 451 -> 360; at 333 rows, down 105 -> 34 us, 30 of it the
-// split over k.  hipBLASLt's fp16 GEMM on the same shapes: 1515, 974, 822.
+// without), out 451 -> 360; at 333 rows, down 106 -> 33 us (83 without the
+// split over k).  hipBLASLt's fp16 GEMM on the same shapes: 1515, 974, 822.
 //
 // Schedule, IT = 4: the waves of wave row 0 (one per SIMD) and of wave row 1
 // (the other one of each SIMD) run half a phase apart.  A phase is 32 k: first
@@ -461,19 +461,23 @@ __global__ __launch_bounds__(512, 1) void w8t_kernel(const uint16_t *__restrict_
 }
 
 // Sums the S parts of every split tile in part order and runs the tile's
-// epilogue, with the multiplying kernel's wave and lane mapping: block
-// (split tile, row tile it of each wave).
+// epilogue, with the multiplying kernel's wave and lane mapping: one wave per
+// block (split tile, 8 it + wave), so that the few tiles of a small problem
+// spread over the chip (with eight waves a block, 30 tiles of 128 rows in 8
+// parts took 8.6 us; 60 tiles of 64 rows in 4 parts take 5.4), kParts parts' loads in flight together.
 template <int IT, int MODE>
-__global__ __launch_bounds__(512) void w8t_reduce_kernel(const float *__restrict__ part,
-                                                         const float *__restrict__ scale, int M, int N,
-                                                         W8tPlan plan, W8Out out) {
-    __shared__ __align__(16) float scratch[8 * kPScratch];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 2, wn = wave & 3, it = blockIdx.y;
+__global__ __launch_bounds__(64) void w8t_reduce_kernel(const float *__restrict__ part,
+                                                        const float *__restrict__ scale, int M, int N,
+                                                        W8tPlan plan, W8Out out) {
+    constexpr int kParts = 4;
+    __shared__ __align__(16) float scratch[kPScratch];
+    const int lane = threadIdx.x;
+    const int wave = blockIdx.y & 7, it = blockIdx.y >> 3;
+    const int wm = wave >> 2, wn = wave & 3;
     int tm, tn;
     w8t_tile(plan, plan.full + blockIdx.x, tm, tn);
     const int nc = tn * kPBN + 64 * wn, row0 = tm * 64 * IT + 32 * (IT * wm + it);
-    if (nc >= N || row0 >= M) return;  // wave-uniform; no barriers below
+    if (nc >= N || row0 >= M) return;
     const float *pp =
         part + ((size_t)blockIdx.x * plan.S * 8 + wave) * (IT * kPPartWave) + it * kPPartWave + lane * 4;
     f32x16_t acc[1][2];
@@ -481,17 +485,23 @@ __global__ __launch_bounds__(512) void w8t_reduce_kernel(const float *__restrict
     for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[0][jt][e] = 0.f;
-    for (int s = 0; s < plan.S; ++s) {
-        f32x4_t y[8];
+    for (int s0 = 0; s0 < plan.S; s0 += kParts) {
+        f32x4_t y[kParts][8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
-            y[q] = *reinterpret_cast<const f32x4_t *>(pp + (size_t)s * 8 * (IT * kPPartWave) + q * 256);
+        for (int s = 0; s < kParts; ++s)
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
+            for (int q = 0; q < 8; ++q)
+                if (s0 + s < plan.S)
+                    y[s][q] = *reinterpret_cast<const f32x4_t *>(pp + (size_t)(s0 + s) * 8 * (IT * kPPartWave) + q * 256);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[0][q >> 2][4 * (q & 3) + e] += y[q][e];
+        for (int s = 0; s < kParts; ++s)
+            if (s0 + s < plan.S)
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[0][q >> 2][4 * (q & 3) + e] += y[s][q][e];
     }
-    w8t_epilogue<1, MODE>(acc, scratch + wave * kPScratch, row0, nc, scale, M, N, out);
+    w8t_epilogue<1, MODE>(acc, scratch, row0, nc, scale, M, N, out);
 }
 
 // ---- causal prefill attention ------------------------------------------------
@@ -724,7 +734,7 @@ constexpr size_t kW8tPartBytes = 384u << 20; // partial sums of one launch at mo
 struct W8tChoice {
     int it = 1;
     W8tPlan plan{};
-    size_t part_bytes = 0;
+    size_t need = 0;  // bytes of partials with which the same split is chosen (any row tile fits them)
 };
 
 W8tPlan w8t_plan(int M, int N, int it, int S, bool tail) {
@@ -756,7 +766,7 @@ double w8t_cost(const W8tPlan &p, int it, int ksteps) {
     double t = rounds * (ksteps * step + it);
     if (split_units > 0) {
         const int parts = (split_units + kW8tBlocks - 1) / kW8tBlocks;
-        t += parts * ((ksteps + p.S - 1) / p.S * step + it) + 4.0 + 2.0 * w8t_part_bytes(p, it) / 4.5e6;
+        t += parts * ((ksteps + p.S - 1) / p.S * step + it) + 3.0 + 2.0 * w8t_part_bytes(p, it) / 4.5e6;
     }
     return t;
 }
@@ -773,6 +783,7 @@ W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, s
     part_limit = std::min(part_limit, kW8tPartBytes);
     const auto it_fits = [&](int it) { return (uint64_t)(8 * it) * ldx * 2 < (1ull << 32); };  // 32-bit row offsets
     int S = 1;
+    size_t need = 0;
     double best = 1e30;
     for (int s = 1; s <= kW8tMaxSplits && (s == 1 || ksteps / s >= kW8tMinSteps); ++s)
         for (int it = 1; it <= 4; it *= 2) {
@@ -784,6 +795,7 @@ W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, s
             if (c < best) {
                 best = c;
                 S = s;
+                need = s > 1 ? w8t_part_bytes(worst, tail ? it : 4) : 0;
             }
         }
     W8tChoice r;
@@ -795,7 +807,7 @@ W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, s
         const double c = w8t_cost(p, it, ksteps);
         if (pb <= part_limit && c < best) {
             best = c;
-            r = W8tChoice{it, p, pb};
+            r = W8tChoice{it, p, need};
         }
     }
     return r;
@@ -806,7 +818,7 @@ hipError_t w8t_run(const uint16_t *x, int ldx, const int8_t *W, const float *sca
                    const W8tPlan &p, float *part, const W8Out &out, hipStream_t st) {
     w8t_kernel<IT, MODE><<<p.grid, 512, 0, st>>>(x, ldx, W, scale, M, N, K, p, part, out);
     const int split = p.tiles_m * p.tiles_n - p.full;
-    if (split > 0) w8t_reduce_kernel<IT, MODE><<<dim3(split, IT), 512, 0, st>>>(part, scale, M, N, p, out);
+    if (split > 0) w8t_reduce_kernel<IT, MODE><<<dim3(split, 8 * IT), 64, 0, st>>>(part, scale, M, N, p, out);
     return hipGetLastError();
 }
 template <int MODE>
@@ -819,7 +831,7 @@ hipError_t w8t_run_it(const W8tChoice &c, const uint16_t *x, int ldx, const int8
 
 }  // namespace
 
-size_t w8p_part_bytes(int M, int N, int K) { return w8t_choose(M, M, M, N, K, K, kW8tPartBytes).part_bytes; }
+size_t w8p_part_bytes(int M, int N, int K) { return w8t_choose(M, M, M, N, K, K, kW8tPartBytes).need; }
 size_t w8p_part_bytes_max() { return kW8tPartBytes; }
 
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
