@@ -102,7 +102,9 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t *tokens, const
 // Qwen3_5RMSNorm (modeling_qwen3_5.py:720-737) with the residual add fused:
 // h += d (when d), out = fp16(h / sqrt(mean(h^2) + eps) * (1 + w)).  One
 // block per row; thread t holds the float4 chunks t, t + 256, ... (H / 4 <=
-// 256 kNormChunks), all loaded before any arithmetic.
+// 256 kNormChunks), all loaded before any arithmetic, the weight's too: at
+// decode sizes the kernel is its load latencies, and after the row's sum the
+// weight would cost a second one.
 constexpr int kNormChunks = 8;
 __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, const float *__restrict__ d,
                                                       const float *__restrict__ w, uint16_t *__restrict__ out,
@@ -111,13 +113,14 @@ __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, con
     const size_t b = blockIdx.x;
     float4 *hr = reinterpret_cast<float4 *>(h + b * H);
     const int n4 = H / 4;
-    float4 x[kNormChunks], dv[kNormChunks];
+    float4 x[kNormChunks], dv[kNormChunks], wv[kNormChunks];
 #pragma unroll
     for (int j = 0; j < kNormChunks; ++j) {
         const int i = threadIdx.x + 256 * j;
         if (i < n4) {
             x[j] = hr[i];
             if (d) dv[j] = reinterpret_cast<const float4 *>(d + b * H)[i];
+            wv[j] = reinterpret_cast<const float4 *>(w)[i];
         }
     }
     float ss = 0.f;
@@ -140,12 +143,11 @@ __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, con
     for (int j = 0; j < kNormChunks; ++j) {
         const int i = threadIdx.x + 256 * j;
         if (i < n4) {
-            const float4 wv = reinterpret_cast<const float4 *>(w)[i];
             uint2 o;
-            o.x = (uint32_t)f32_to_f16_rne(x[j].x * inv * (1.0f + wv.x)) |
-                  ((uint32_t)f32_to_f16_rne(x[j].y * inv * (1.0f + wv.y)) << 16);
-            o.y = (uint32_t)f32_to_f16_rne(x[j].z * inv * (1.0f + wv.z)) |
-                  ((uint32_t)f32_to_f16_rne(x[j].w * inv * (1.0f + wv.w)) << 16);
+            o.x = (uint32_t)f32_to_f16_rne(x[j].x * inv * (1.0f + wv[j].x)) |
+                  ((uint32_t)f32_to_f16_rne(x[j].y * inv * (1.0f + wv[j].y)) << 16);
+            o.y = (uint32_t)f32_to_f16_rne(x[j].z * inv * (1.0f + wv[j].z)) |
+                  ((uint32_t)f32_to_f16_rne(x[j].w * inv * (1.0f + wv[j].w)) << 16);
             reinterpret_cast<uint2 *>(out + b * H)[i] = o;
         }
     }
