@@ -520,7 +520,13 @@ GDN_DEV int vt_slot(int d, int c) { return d * kApK + ((c ^ (d & 7)) << 3); }
 // that share every K and V fragment the wave reads from LDS (two MFMAs per
 // fragment read, against one with a tile per wave: the LDS reads bounded
 // that form).  K (the cache's tiled layout, 32 KB per step, contiguous) and
-// V^T (from the transposed copy) reach LDS by DMA, double buffered.
+// V^T (from the transposed copy) reach LDS by DMA, double buffered.  The DMA
+// is dma16's: as a builtin on one two-slot array the compiler waited for the
+// next step's tiles before this step's first LDS read, and so did queries
+// still in flight at the loop (20000 positions: 4.39 -> 4.12 ms a layer, 0.80
+// PFLOP/s counting the causal half).  What bounds it now: two waves per SIMD
+// whose LDS reads, MFMAs and softmax hide each other only in part (running
+// the two position halves half a phase apart, as the GEMM does, took 4.26).
 constexpr int kApT = 2;  // query tiles per wave
 constexpr int kApThreads = 512;
 
@@ -582,20 +588,16 @@ __global__ __launch_bounds__(kApThreads) void attn_prefill_kernel(
     // per-lane parts of the DMA addresses (loop-invariant): K chunk lane of a
     // kilobyte; V^T row lane / 8 of an 8-row group (whose first row is a
     // multiple of 8, so the row's swizzle is (lane / 8) % 8), piece lane % 8
-    const int koff = lane * 8;
-    const int voff = (lane >> 3) * Tv + 8 * ((lane & 7) ^ (lane >> 3));
+    const uint32_t koff = lane * 16, voff = 2u * ((lane >> 3) * (uint32_t)Tv + 8 * ((lane & 7) ^ (lane >> 3)));
+    const uint32_t kl = lds_addr(ks) + 4096u * wave, vl = lds_addr(vs) + 4096u * wave;
     auto dma = [&](int kb, int b) {
         const int t0 = min(kb * kApK + 16 * (wave >> 1), Tmax - 16);
         const uint16_t *kp = kbase + (size_t)t0 * kApD + (4 * (wave & 1)) * 512;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds(kp + i * 512 + koff, (lds_void_t *)&ks[b][(4 * wave + i) * 512], 16, 0,
-                                             0);
+        for (int i = 0; i < 4; ++i) dma16(kp + i * 512, koff, kl + 32768u * b + 1024u * i);
         const uint16_t *vp = vbase + (size_t)(32 * wave) * Tv + kb * kApK;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds(vp + (size_t)(8 * i) * Tv + voff,
-                                             (lds_void_t *)&vs[b][(32 * wave + 8 * i) * kApK], 16, 0, 0);
+        for (int i = 0; i < 4; ++i) dma16(vp + (size_t)(8 * i) * Tv, voff, vl + 32768u * b + 1024u * i);
     };
     // One step: the 64 keys of buffer b as two halves of 32, each an online
     // softmax update (scores, P, then P V), so that one half's scores and P
@@ -685,12 +687,18 @@ __global__ __launch_bounds__(kApThreads) void attn_prefill_kernel(
 
     dma(0, 0);
     wait_vm<0>();
-    __syncthreads();
+    lds_bar();
+    // the queries land here: waited for at their first use, every step would
+    // wait for its own prefetch
+#pragma unroll
+    for (int qt = 0; qt < kApT; ++qt)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) __asm__ volatile("" : "+v"(qf[qt][j]));
     for (int kb = 0; kb < nkb; ++kb) {
         if (kb + 1 < nkb) dma(kb + 1, (kb + 1) & 1);  // into the buffer step kb - 1 read
         step(kb & 1, kb);
         wait_vm<0>();
-        __syncthreads();
+        lds_bar();
     }
     if (!live) return;
 #pragma unroll
