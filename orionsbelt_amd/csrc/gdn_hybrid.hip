@@ -102,10 +102,12 @@ __global__ __launch_bounds__(256) void embed_kernel(const int32_t *tokens, const
 // Qwen3_5RMSNorm (modeling_qwen3_5.py:720-737) with the residual add fused:
 // h += d (when d), out = fp16(h / sqrt(mean(h^2) + eps) * (1 + w)).  One
 // block per row; thread t holds the float4 chunks t, t + 256, ... (H / 4 <=
-// 256 kNormChunks), all loaded before any arithmetic, the weight's too: at
-// decode sizes the kernel is its load latencies, and after the row's sum the
-// weight would cost a second one.
+// 256 kNormChunks), all loaded before any arithmetic.  FEW: the weight's too:
+// at decode sizes the kernel is its load latencies, and after the row's sum
+// the weight would cost a second one (4 rows: 3.84 -> 3.52 us); with the chip
+// full the registers it holds cost more (32768 rows: 88 -> 119 us).
 constexpr int kNormChunks = 8;
+template <bool FEW>
 __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, const float *__restrict__ d,
                                                       const float *__restrict__ w, uint16_t *__restrict__ out,
                                                       int H, float eps) {
@@ -113,14 +115,14 @@ __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, con
     const size_t b = blockIdx.x;
     float4 *hr = reinterpret_cast<float4 *>(h + b * H);
     const int n4 = H / 4;
-    float4 x[kNormChunks], dv[kNormChunks], wv[kNormChunks];
+    float4 x[kNormChunks], dv[kNormChunks], wv[FEW ? kNormChunks : 1];
 #pragma unroll
     for (int j = 0; j < kNormChunks; ++j) {
         const int i = threadIdx.x + 256 * j;
         if (i < n4) {
             x[j] = hr[i];
             if (d) dv[j] = reinterpret_cast<const float4 *>(d + b * H)[i];
-            wv[j] = reinterpret_cast<const float4 *>(w)[i];
+            if constexpr (FEW) wv[j] = reinterpret_cast<const float4 *>(w)[i];
         }
     }
     float ss = 0.f;
@@ -143,14 +145,21 @@ __global__ __launch_bounds__(256) void addnorm_kernel(float *__restrict__ h, con
     for (int j = 0; j < kNormChunks; ++j) {
         const int i = threadIdx.x + 256 * j;
         if (i < n4) {
+            const float4 ww = FEW ? wv[FEW ? j : 0] : reinterpret_cast<const float4 *>(w)[i];
             uint2 o;
-            o.x = (uint32_t)f32_to_f16_rne(x[j].x * inv * (1.0f + wv[j].x)) |
-                  ((uint32_t)f32_to_f16_rne(x[j].y * inv * (1.0f + wv[j].y)) << 16);
-            o.y = (uint32_t)f32_to_f16_rne(x[j].z * inv * (1.0f + wv[j].z)) |
-                  ((uint32_t)f32_to_f16_rne(x[j].w * inv * (1.0f + wv[j].w)) << 16);
+            o.x = (uint32_t)f32_to_f16_rne(x[j].x * inv * (1.0f + ww.x)) |
+                  ((uint32_t)f32_to_f16_rne(x[j].y * inv * (1.0f + ww.y)) << 16);
+            o.y = (uint32_t)f32_to_f16_rne(x[j].z * inv * (1.0f + ww.z)) |
+                  ((uint32_t)f32_to_f16_rne(x[j].w * inv * (1.0f + ww.w)) << 16);
             reinterpret_cast<uint2 *>(out + b * H)[i] = o;
         }
     }
+}
+hipError_t addnorm(int rows, float *h, const float *d, const float *w, uint16_t *out, int H, float eps,
+                   hipStream_t st) {
+    if (rows <= 512) addnorm_kernel<true><<<rows, 256, 0, st>>>(h, d, w, out, H, eps);  // two blocks per CU
+    else addnorm_kernel<false><<<rows, 256, 0, st>>>(h, d, w, out, H, eps);
+    return hipGetLastError();
 }
 
 // Attention prologue (Qwen3_5Attention.forward:656-681): block (slot, row),
@@ -665,8 +674,7 @@ hipError_t gemm_addnorm(kai_gdn_hybrid *m, const uint16_t *x, const Mat &w, floa
         return hipSuccess;
     }
     TRY(gemm_to(m, x, w, d, H, st));
-    addnorm_kernel<<<B, 256, 0, st>>>(m->h, d, norm_w, m->x16, H, m->cfg.rms_eps);
-    return hipGetLastError();
+    return addnorm(B, m->h, d, norm_w, m->x16, H, m->cfg.rms_eps, st);
 }
 
 // o = norm(h) W^T: from x16, or, at batch 1, normalising the residual
@@ -832,8 +840,7 @@ hipError_t step(kai_gdn_hybrid *m, const int32_t *tokens, int32_t *next, float *
     m->hnext = m->h2;
     m->pend_w = m->layers[0].ln_in;
     if (!norm_in(m)) {
-        addnorm_kernel<<<B, 256, 0, st>>>(m->h, nullptr, m->layers[0].ln_in, m->x16, H, c.rms_eps);
-        TRY(hipGetLastError());
+        TRY(addnorm(B, m->h, nullptr, m->layers[0].ln_in, m->x16, H, c.rms_eps, st));
     }
     TRY(mark(m, KAI_GDN_PHASE_OTHER, st));
     for (size_t l = 0; l < m->layers.size(); ++l) {
@@ -942,8 +949,7 @@ hipError_t prefill_group(kai_gdn_hybrid *m, const int32_t *tokens, int b0, Rows 
     TRY(mark(m, -1, st));
     embed_kernel<<<R, 256, 0, st>>>(tokens, m->embed, p.h, H, c.vocab);
     TRY(hipGetLastError());
-    addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, m->layers[0].ln_in, p.x16, H, c.rms_eps);
-    TRY(hipGetLastError());
+    TRY(addnorm(R, p.h, nullptr, m->layers[0].ln_in, p.x16, H, c.rms_eps, st));
     TRY(hipMemsetAsync(p.hist, 0, (size_t)3 * C * sizeof(float), st));
     TRY(mark(m, KAI_GDN_PHASE_OTHER, st));
     W8Out swiglu{};
@@ -991,13 +997,11 @@ hipError_t prefill_group(kai_gdn_hybrid *m, const int32_t *tokens, int b0, Rows 
             TRY(w8p_residual(m, p.x16, Hq * 256, L.out, r, p.h, H, st));
             TRY(mark(m, KAI_GDN_PHASE_ATTN, st));
         }
-        addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, L.ln_post, p.x16, H, c.rms_eps);
-        TRY(hipGetLastError());
+        TRY(addnorm(R, p.h, nullptr, L.ln_post, p.x16, H, c.rms_eps, st));
         TRY(w8p(m, p.x16, H, L.gate_up, r, swiglu, st));
         TRY(w8p_residual(m, p.act16, I, L.down, r, p.h, H, st));
         const float *next_norm = l + 1 < m->layers.size() ? m->layers[l + 1].ln_in : m->final_norm;
-        addnorm_kernel<<<R, 256, 0, st>>>(p.h, nullptr, next_norm, p.x16, H, c.rms_eps);
-        TRY(hipGetLastError());
+        TRY(addnorm(R, p.h, nullptr, next_norm, p.x16, H, c.rms_eps, st));
         TRY(mark(m, KAI_GDN_PHASE_FFN, st));
     }
     last_rows_kernel<<<r.nseq, 256, 0, st>>>(p.x16, m->x16 + (size_t)b0 * H, T, H);

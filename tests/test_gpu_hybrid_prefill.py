@@ -179,6 +179,7 @@ def test_prefill_rows_independent_and_replayable(hb, fixture):
 
 
 @pytest.mark.parametrize("T,batch", [(1, 4), (70, 4),  # one group; GEMMs with k-splits
+                                     (300, 4),          # norm rows on both sides of the few-rows form
                                      (704, 4),          # the longest prompt whose delta rule runs grouped
                                      (705, 3),          # and the shortest one run per sequence
                                      (1400, 4)])        # two sequences per group
