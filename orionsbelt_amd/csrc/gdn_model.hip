@@ -742,17 +742,23 @@ hipError_t launch_w8f(const uint16_t *x, const int8_t *W, const float *scale, in
 // head h of sequence b, with kv = h / (Hq / Hkv) (repeat_kv),
 //   o[b][h] = softmax_t(scaling * q[b][h] . K[b][kv][t]) . V[b][kv][t],  t < L
 // q [B][Hq][256] fp16, K, V [B][Hkv][Tmax][256] fp16, fp32 softmax and sums.
-// Split over the sequence: block (span, kv, b) takes 64 G consecutive
-// positions (attn_groups) and every query head of kv; wave w takes 16 G of
-// them in groups of 16.  Scores on fp16 MFMA 16x16x32 (A = 16 key rows, B = the
+// Split over the sequence: block (span, kv, b) takes a span of at most 64 G
+// positions (attn_groups) and every query head of kv, each wave up to G
+// groups of 16.  Scores on fp16 MFMA 16x16x32 (A = 16 key rows, B = the
 // group's query heads as columns); online softmax per head in exp2; P.V on
 // the VALU, lane l holding dims 4l .. 4l+3 of every head's output.  The
 // block's four waves merge through LDS into one partial (max, sum, o) per
 // head; attn_combine_kernel merges the spans.  With a tiled K cache (the
 // hybrid model's own) each group's 16 rows are 8 contiguous KB laid out in
-// MFMA-lane order, so every K load of a wave is one contiguous 1 KB (10%
-// faster at B=16 and 32K than the 16 x 64-byte row pieces of the row-major
-// cache).
+// MFMA-lane order, so every K load of a wave is one contiguous 1 KB.
+// A row-major cache is read the same way, two whole rows a load, and the rows
+// reach operand order through LDS: loaded straight into operand order a load
+// takes 64 bytes of each of 16 rows, and needs cached loads to use a line's
+// other half (non-temporal, B = 8 at 12289 88 us against 79 cached and 75 this
+// way); cached loads in turn evict what the last-level cache still has to
+// write back, and a first pass over a cache just written paid for it (B = 16
+// at 32K: 454 us cached, 412 non-temporal, 396 this way; B = 64 at 3000: 189,
+// 162, 149).
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -764,12 +770,13 @@ constexpr int kAttPart = kAttD + 2;
 
 template <bool KTILED>
 __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__restrict__ q,
-                                                          const uint16_t *__restrict__ Kc,
-                                                          const uint16_t *__restrict__ Vc,
-                                                          float *__restrict__ part, int Hq, int Hkv,
-                                                          int Tmax, int L, int nspan, int G, float sc_log2) {
+                                                             const uint16_t *__restrict__ Kc,
+                                                             const uint16_t *__restrict__ Vc,
+                                                             float *__restrict__ part, int Hq, int Hkv,
+                                                             int Tmax, int L, int nspan, int G, float sc_log2) {
     __shared__ float s_m[4][kAttRepMax], s_l[4][kAttRepMax];
     __shared__ float s_o[4][kAttRepMax][kAttD];
+    __shared__ __align__(16) uint16_t s_k[KTILED ? 1 : 4][KTILED ? 8 : 16 * kAttD];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, r = lane & 15;
     const int span = blockIdx.x, kv = blockIdx.y, b = blockIdx.z;
@@ -792,12 +799,16 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__r
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[h][i] = 0.f;
     }
-    // Each wave takes G groups of 16 positions (the span is 64 G),
-    // double-buffered: the K rows and V rows of the next group are in
-    // flight while a group is scored and accumulated.  Rows past L are
-    // clamped to L - 1 (in bounds; masked by p = 0).
-    const int t_begin = span * (64 * G) + wave * (16 * G);
-    const int t_end = min(t_begin + 16 * G, L);
+    // Each wave takes up to G groups of 16 positions, double-buffered: the K
+    // rows and V rows of the next group are in flight while a group is scored
+    // and accumulated.  Rows past L are clamped to L - 1 (in bounds; masked by
+    // p = 0).  KTILED: a span is 64 G consecutive positions, a wave's groups
+    // follow each other.  Row-major: the spans' groups interleave, so that the
+    // blocks of a (sequence, kv head) walk its rows together (B = 16 at 32K:
+    // 355 us against 364 with consecutive spans).
+    const int t_begin = KTILED ? span * (64 * G) + wave * (16 * G) : (span * 4 + wave) * 16;
+    const int t_step = KTILED ? 16 : nspan * 64;
+    const int t_end = KTILED ? min(t_begin + 16 * G, L) : L;
     u32x4_t kbuf[2][8];
     u32x2_t vbuf[2][16];
     auto load_group = [&](int t0, u32x4_t (&kb)[8], u32x2_t (&vb)[16]) {
@@ -808,12 +819,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__r
             for (int j = 0; j < 8; ++j)
                 kb[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(kp + 512 * j));
         } else {
-            // cached loads: a row's 64-byte pieces of two loads share a 128-byte
-            // line (non-temporal, 8 x 12289 positions take 88 us instead of 78;
-            // V's whole 512-byte rows are faster non-temporal, 78 against 85)
-            const uint16_t *kp = Kc + (kvrow + min(t0 + r, L - 1)) * kAttD + 8 * g;
+            // two whole rows per load (instruction i: rows 2i, 2i + 1)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) kb[j] = *reinterpret_cast<const u32x4_t *>(kp + 32 * j);
+            for (int i = 0; i < 8; ++i)
+                kb[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(
+                    Kc + (kvrow + min(t0 + 2 * i + (lane >> 5), L - 1)) * kAttD + 8 * (lane & 31)));
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i)
@@ -821,10 +831,30 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__r
                 reinterpret_cast<const u32x2_t *>(Vc + (kvrow + min(t0 + i, L - 1)) * kAttD + 4 * lane));
     };
     auto process = [&](const u32x4_t (&kb)[8], const u32x2_t (&vb)[16], int t0) {
+        u32x4_t ka[8];  // A operand: row r, dims 32 j + 8 g .. +7
+        if constexpr (KTILED) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ka[j] = kb[j];
+        } else {
+            // rows to operand order through the wave's own LDS: 16-byte piece
+            // p of row t in slot p ^ (t % 8), so that the eight rows a read
+            // takes at once cover all banks
+            uint16_t *ks = s_k[wave];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int t = 2 * i + (lane >> 5);
+                *reinterpret_cast<u32x4_t *>(ks + t * kAttD + (((lane & 31) ^ (t & 7)) << 3)) = kb[i];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                ka[j] = *reinterpret_cast<const u32x4_t *>(ks + r * kAttD + (((4 * j + g) ^ (r & 7)) << 3));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
         f32x4_t acc = zero4();
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, kb[j]), qb[j], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, ka[j]), qb[j], acc, 0, 0, 0);
         // lane (g, r): scores of positions t0 + 4g + e for head r, in log2 units
         float s[4];
 #pragma unroll
@@ -886,12 +916,12 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const uint16_t *__r
         }
     };
     if (t_begin < t_end) load_group(t_begin, kbuf[0], vbuf[0]);
-    for (int t0 = t_begin; t0 < t_end; t0 += 32) {  // uniform over the wave
-        const int t1 = t0 + 16;
+    for (int t0 = t_begin; t0 < t_end; t0 += 2 * t_step) {  // uniform over the wave
+        const int t1 = t0 + t_step;
         if (t1 < t_end) load_group(t1, kbuf[1], vbuf[1]);
         process(kbuf[0], vbuf[0], t0);
         if (t1 >= t_end) break;
-        if (t1 + 16 < t_end) load_group(t1 + 16, kbuf[0], vbuf[0]);
+        if (t1 + t_step < t_end) load_group(t1 + t_step, kbuf[0], vbuf[0]);
         process(kbuf[1], vbuf[1], t1);
     }
     // merge the four waves (each may have seen no position: m = -inf, l = 0)
@@ -993,12 +1023,15 @@ namespace {
 // blocks: at B = 16 and 32K, spans of 16 groups (2112 blocks) took 356.5
 // against 381.4 us per layer with 4 groups (8256 blocks), decode and combine,
 // with 8 to 24 groups all within 364 us (longer spans read the KV stream
-// faster and leave fewer partials to combine).  Row-major caches, against
-// spans of 256 positions always: B = 8 at 12289 88 -> 78 us, B = 16 at 32K
-// 405 -> 364, B = 4 at 4096 23.2 -> 19.8, B = 1 at 2000 20.4 -> 9.6.
-int attn_groups(int B, int Hkv, int L) {
+// faster and leave fewer partials to combine).  A large row-major grid is cut
+// into about 4096: a first pass over a cache just written is slower with
+// longer spans (B = 16 at 32K: 397 us at 4096 blocks, 417 at 2048, 390 at
+// 8192; read again 356, 345 and 383).  Against spans of 256 positions
+// and half-line loads always: B = 8 at 12289 88 -> 75 us, B = 16 at 32K 408
+// -> 356, B = 4 at 4096 22.3 -> 18.8, B = 1 at 2000 19.2 -> 9.1.
+int attn_groups(int B, int Hkv, int L, bool k_tiled) {
     const long long pairs = (long long)B * Hkv, blocks256 = pairs * ((L + kAttSpan - 1LL) / kAttSpan);
-    const long long target = blocks256 >= 2048 ? 2048 : 512, per_kv = std::max(1LL, target / pairs);
+    const long long target = blocks256 < 2048 ? 512 : k_tiled ? 2048 : 4096, per_kv = std::max(1LL, target / pairs);
     return (int)((L + 64 * per_kv - 1) / (64 * per_kv));
 }
 size_t span_bytes(int B, int Hq, int nspan) { return (size_t)B * Hq * nspan * kAttPart * sizeof(float); }
@@ -1010,7 +1043,7 @@ size_t attn_workspace_bytes(int B, int Hq, int L) {
     int nspan = (L + kAttSpan - 1) / kAttSpan;
     for (int rep = 1; rep <= kAttRepMax; ++rep)
         if (Hq % rep == 0) {
-            const int G = attn_groups(B, Hq / rep, L);
+            const int G = attn_groups(B, Hq / rep, L, false);
             nspan = max(nspan, (int)((L + 64LL * G - 1) / (64LL * G)));
         }
     return span_bytes(B, Hq, nspan);
@@ -1031,7 +1064,7 @@ hipError_t launch_attn_decode(const uint16_t *q, const uint16_t *Kc, const uint1
     const size_t fit = workspace_bytes / span_bytes(B, Hq, 1);
     if (fit == 0) return hipErrorInvalidValue;
     const int cap = (int)std::min<size_t>(fit, 1u << 24);
-    const int G = max(attn_groups(B, Hkv, L), (int)((L + 64LL * cap - 1) / (64LL * cap)));
+    const int G = max(attn_groups(B, Hkv, L, k_tiled), (int)((L + 64LL * cap - 1) / (64LL * cap)));
     const int nspan = (L + 64 * G - 1) / (64 * G);
     const float sc_log2 = scaling * 1.4426950408889634f;
     if (k_tiled)

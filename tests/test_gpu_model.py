@@ -266,7 +266,9 @@ def test_attn_decode_peaked_and_long(L):
 @pytest.mark.parametrize("B,Hq,Hkv,length", [(1, 4, 1, 17), (3, 16, 4, 63), (2, 8, 8, 65), (1, 16, 4, 257),
                                              (5, 6, 2, 1000), (1, 16, 4, 4097),
                                              (64, 16, 4, 2100),   # more than 2048 blocks of 256 positions
-                                             (130, 16, 4, 70)])   # more (sequence, kv head) pairs than blocks wanted
+                                             (130, 16, 4, 70),    # more (sequence, kv head) pairs than blocks wanted
+                                             (300, 2, 2, 700),    # one block per pair: eleven groups a wave
+                                             (260, 8, 8, 257)])   # more than 2048 blocks, two groups a wave, one position over
 def test_attn_decode_span_rule(L, B, Hq, Hkv, length):
     """Spans sized by the grid (the queried workspace) and the longest spans
     (the least workspace accepted), against 64-bit attention.  Bound per
