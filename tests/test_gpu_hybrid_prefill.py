@@ -35,6 +35,8 @@ twice what was measured on MI355X:
       (measured 7.0e-4); the whole 4B model, prefill of T then a step against
       a prefill of T + 1: 3e-2 (measured 1.4e-2).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -199,6 +201,59 @@ def test_prefill_groups_match_single_prompts(hb, T, batch):
         for got, want in zip(alone, rows):
             assert np.array_equal(got[0].view(np.uint32), want[b].view(np.uint32)), (T, b)
     gm.close()
+
+
+class _W8Seg(ctypes.Structure):
+    _fields_ = [("dst", ctypes.c_void_p), ("ld", ctypes.c_int), ("n_end", ctypes.c_int)]
+
+
+class _W8Out(ctypes.Structure):  # gdn_internal.h
+    _fields_ = [("seg", _W8Seg * 4), ("nseg", ctypes.c_int), ("mode", ctypes.c_int), ("x16", ctypes.c_void_p),
+                ("nin_h", ctypes.c_void_p), ("nin_add", ctypes.c_void_p), ("nin_hout", ctypes.c_void_p),
+                ("nin_w", ctypes.c_void_p), ("nin_eps", ctypes.c_float), ("add_in", ctypes.c_void_p),
+                ("add_ld", ctypes.c_int)]
+
+
+@pytest.mark.parametrize("M", [17, 130, 600])  # row tiles of 64, 128 and 256
+def test_prefill_swiglu_precision(hb, M):
+    """The prefill GEMM's SwiGLU epilogue (gdn::launch_w8p) on chosen gate and
+    up values (each the channel's scale: one weight and one activation are 1),
+    against 64 bits.  Bound before the fp16 rounding: one ulp each for expf's
+    result, 1 + e, the quotient and the product with up, 4 x 2^-23; the fp16
+    result lies between the roundings of the bound's two ends."""
+    import orionsbelt_amd as ob
+    torch = torch_mod()
+    L = ob.lib()
+    fn = L._ZN3gdn10launch_w8pEPKtiPKaPKfiiiiiRKNS_5W8OutEPfmP12ihipStream_t
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int] * 5 + [
+        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    I, K = 1 << 16, 256
+    rs = np.random.RandomState(M)
+    gate = rs.uniform(-80, 20, I).astype(np.float32)
+    t = gate.astype(np.float64) / (1 + np.exp(-gate.astype(np.float64)))
+    up = (rs.uniform(1, 2, I) * 2.0 ** -np.floor(np.log2(np.abs(t)))).astype(np.float32)  # results in 1 .. 4
+    gate[:6] = np.inf, 3e38, 2.4e38, -3e38, -1000.0, 0.0
+    up[:6] = 1.0, 1e-36, 1e-36, 1.0, 1.0, 1.0
+    scale = np.empty((I // 8, 2, 8), np.float32)  # groups of 8 gate channels, then their 8 up channels
+    scale[:, 0], scale[:, 1] = gate.reshape(-1, 8), up.reshape(-1, 8)
+    w = torch.zeros(2 * I, K, dtype=torch.int8, device="cuda")
+    w[:, 0] = 1
+    wt = torch.empty_like(w)
+    st = torch.cuda.current_stream().cuda_stream
+    assert L.kai_run_gdn_w8_tile_hip(w.data_ptr(), wt.data_ptr(), 2 * I, K, st) == 0
+    x = torch.zeros(M, K, dtype=torch.float16, device="cuda")
+    x[:, 0] = 1
+    sc = torch.from_numpy(scale.reshape(-1)).cuda()
+    y = torch.empty(M, I, dtype=torch.float16, device="cuda")
+    o = _W8Out(mode=1, x16=y.data_ptr())
+    assert fn(x.data_ptr(), K, wt.data_ptr(), sc.data_ptr(), M, M, M, 2 * I, K, ctypes.byref(o), None, 0, st) == 0
+    got = y.cpu().numpy()
+    assert np.array_equal(got.view(np.uint16), np.broadcast_to(got[:1], got.shape).view(np.uint16))
+    with np.errstate(over="ignore"):
+        t = gate.astype(np.float64) / (1 + np.exp(-gate.astype(np.float64))) * up
+        ends = np.stack([t * (1 - 4 * 2.0 ** -23), t * (1 + 4 * 2.0 ** -23)]).astype(np.float16)
+    bad = ~((got[0] >= ends.min(0)) & (got[0] <= ends.max(0)))
+    assert not bad.any(), (int(bad.sum()), gate[bad][:4], got[0][bad][:4])
 
 
 def test_prefill_rejects_bad_arguments(hb, fixture):
