@@ -80,8 +80,9 @@ int kai_gdn_hybrid_step(kai_gdn_hybrid *m, const int32_t *tokens, int32_t *next,
  * max_context.  Prompts that fit 4096 rows together run as one group; a
  * sequence's results do not depend on the others.  The first call allocates
  * the prefill's activation buffers for max_context positions (or, if more, one
- * group) and 384 MB of scratch (freed by kai_gdn_hybrid_destroy).  The
- * reference e2e program's --prefill mode runs its prompt the same way
+ * group) and the scratch its matrices' k-splits use (at most 384 MB; where
+ * that cannot be had they run unsplit, slower), freed by
+ * kai_gdn_hybrid_destroy.  The reference e2e program's --prefill mode runs its prompt the same way
  * (gdn_e2e_decode.c:2644-2700, with the M > 1 GEMM of :606-612). */
 int kai_gdn_hybrid_prefill(kai_gdn_hybrid *m, const int32_t *tokens, int batch, int length,
                            int32_t *next, float *logits, void *stream);

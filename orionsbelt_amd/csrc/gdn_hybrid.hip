@@ -490,7 +490,8 @@ struct kai_gdn_hybrid {
     // (of one sequence or of several short ones)
     struct Prefill {
         int rows = 0;
-        float *part = nullptr;  // k-split partials of the GEMMs, w8p_part_bytes_max() bytes
+        float *part = nullptr;  // k-split partials of the GEMMs (null: no room for them, no splits)
+        size_t part_bytes = 0;
         float *h = nullptr, *qkv = nullptr, *z = nullptr, *a = nullptr, *b = nullptr;
         float *g = nullptr, *beta = nullptr, *kx = nullptr, *vx = nullptr, *hist = nullptr;
         uint16_t *x16 = nullptr, *act16 = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *o = nullptr;
@@ -873,6 +874,37 @@ constexpr int kPrefillGroupRows = 4096;
 // segments, and with them their roundings, do not depend on the batch.
 constexpr int kPrefillGroupChunks = 11;
 
+// Sequences of T rows that run as one group at most (whatever the batch).
+int group_limit(const kai_gdn_hybrid *m, int T) {
+    return std::max(1, std::min(m->cfg.max_batch, kPrefillGroupRows / T));
+}
+
+// Bytes of k-split partials that the model's prompts use: the most over its
+// matrices and prompt lengths.  A split follows from a prompt's count of
+// 64-row tiles and its group's rows, so the last length of each such step is
+// taken; from kPrefillGroupRows rows only the tiles left over by rounds of 256
+// blocks are split, whose counts repeat every 256 * 256 rows.
+size_t prefill_part_bytes(const kai_gdn_hybrid *m) {
+    const Layer *gdn = nullptr, *attn = nullptr;
+    for (const Layer &L : m->layers) (L.attn ? attn : gdn) = &L;
+    const int last = m->cfg.max_context - 1;
+    size_t bytes = 0;
+    auto take = [&](int T) {
+        const int rows = group_limit(m, T) * T;
+        auto use = [&](const Mat &w) { bytes = std::max(bytes, w8p_part_bytes(T, rows, w.N, w.K)); };
+        for (const Layer *L : {gdn, attn})
+            if (L) {
+                use(L->in);
+                use(L->out);
+            }
+        use(m->layers[0].gate_up);
+        use(m->layers[0].down);
+    };
+    for (int T = 64; T <= std::min(last, kPrefillGroupRows + 256 * 256); T += 64) take(T);
+    for (int n = 1; n <= m->cfg.max_batch; ++n) take(std::max(1, std::min(last, kPrefillGroupRows / n)));
+    return bytes;
+}
+
 hipError_t prefill_alloc(kai_gdn_hybrid *m) {
     if (m->pf.rows) return hipSuccess;
     const kai_gdn_hybrid_config &c = m->cfg;
@@ -901,7 +933,12 @@ hipError_t prefill_alloc(kai_gdn_hybrid *m) {
     TRY(alloc_t(m, &p.o, R * V));
     TRY(alloc_t(m, &p.q16, R * Hq * 256));
     TRY(alloc_t(m, &p.vT, vt));
-    TRY(alloc(m, reinterpret_cast<void **>(&p.part), w8p_part_bytes_max()));
+    p.part_bytes = prefill_part_bytes(m);
+    if (p.part_bytes && alloc(m, reinterpret_cast<void **>(&p.part), p.part_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        p.part = nullptr;
+        p.part_bytes = 0;
+    }
     p.rows = (int)R;
     return hipDeviceSynchronize();
 }
@@ -911,13 +948,9 @@ struct Rows {
     int nseq, T;
     int total() const { return nseq * T; }
 };
-// Sequences of T rows that run as one group at most (whatever the batch).
-int group_limit(const kai_gdn_hybrid *m, int T) {
-    return std::max(1, std::min(m->cfg.max_batch, kPrefillGroupRows / T));
-}
 hipError_t w8p(kai_gdn_hybrid *m, const uint16_t *x, int ldx, const Mat &w, Rows r, const W8Out &o, hipStream_t st) {
     return launch_w8p(x, ldx, w.q, w.s, r.total(), r.T, group_limit(m, r.T) * r.T, w.N, w.K, o, m->pf.part,
-                      w8p_part_bytes_max(), st);
+                      m->pf.part_bytes, st);
 }
 // A branch matrix: h[t] += x[t] W^T for the rows, the residual add in the
 // GEMM's epilogue (in place), so no branch array is written and read back.

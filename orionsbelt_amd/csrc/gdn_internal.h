@@ -200,9 +200,9 @@ hipError_t launch_w8_quantize(const float *W, int8_t *Wq, float *scale, int N, i
 // splits run.
 // The largest M launch_w8p accepts.
 long long w8p_max_rows();
-// Scratch the best split of M rows (one sequence) uses, and the most any uses.
-size_t w8p_part_bytes(int M, int N, int K);
-size_t w8p_part_bytes_max();
+// Scratch the best split of sequences of seq_rows rows, max_rows in all at
+// most, uses.
+size_t w8p_part_bytes(int seq_rows, int max_rows, int N, int K);
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
                       int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st);
 // Causal attention of nseq sequences of T positions, every array with the

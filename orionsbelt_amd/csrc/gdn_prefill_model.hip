@@ -835,8 +835,9 @@ hipError_t w8t_run_it(const W8tChoice &c, const uint16_t *x, int ldx, const int8
 
 }  // namespace
 
-size_t w8p_part_bytes(int M, int N, int K) { return w8t_choose(M, M, M, N, K, K, kW8tPartBytes).need; }
-size_t w8p_part_bytes_max() { return kW8tPartBytes; }
+size_t w8p_part_bytes(int seq_rows, int max_rows, int N, int K) {
+    return w8t_choose(max_rows, seq_rows, max_rows, N, K, K, kW8tPartBytes).need;
+}
 
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
                       int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st) {

@@ -824,7 +824,7 @@ static size_t w8p_ws_tail(int N) { return ((size_t)(N / 64) * sizeof(uint32_t) +
 extern "C" size_t kai_gdn_w8a16_gemm_tiled_workspace_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || N % 64 || K % 256) return 0;
     if (M <= 16) return w8f_ws_bytes(M, N, K);
-    const size_t part = gdn::w8p_part_bytes(M, N, K);
+    const size_t part = gdn::w8p_part_bytes(M, M, N, K);
     return part ? kW8pWsSkip + part + w8p_ws_tail(N) : 0;
 }
 

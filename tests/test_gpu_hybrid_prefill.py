@@ -256,6 +256,23 @@ def test_prefill_swiglu_precision(hb, M):
     assert not bad.any(), (int(bad.sum()), gate[bad][:4], got[0][bad][:4])
 
 
+def test_prefill_memory_follows_the_model(hb):
+    """The first prefill allocates activation rows and k-split scratch for the
+    model's own shapes: per position the row arrays (at most 4 bytes for each
+    of the in-projection's channels, twice that for the rest), and partial
+    sums of at most eight splits of the largest matrix's padded rows."""
+    cfg = dict(layers=2, attn_every=2, hidden=256, inter=512, vocab=512, gdn_k_heads=2, gdn_v_heads=16,
+               attn_q_heads=2, attn_kv_heads=1, max_batch=2, max_context=300, rope_theta=1.0e7, rms_eps=1e-6)
+    gm = hb.HybridModel(hb.config(**cfg), 3)
+    before = gm.device_bytes
+    prefill(gm, np.zeros((2, 200), np.int32), cfg["vocab"])
+    grown = gm.device_bytes - before
+    widest = 2 * 2 * 128 + 2 * 16 * 128 + 2 * 16  # [qkv | z | b | a]
+    rows = 600                                     # both sequences' positions
+    assert grown <= rows * widest * 4 * 3 + 8 * 768 * (widest + 256) * 4, grown
+    gm.close()
+
+
 def test_prefill_rejects_bad_arguments(hb, fixture):
     import orionsbelt_amd as ob
     torch = torch_mod()
