@@ -27,6 +27,7 @@
 // 16 + 4g .. 16 + 4g+3, permute the k index of both operands alike).  Each K
 // and V fragment read from LDS feeds both query tiles.
 #include <algorithm>
+#include <climits>
 
 #include "gdn_common.h"
 #include "gdn_internal.h"
@@ -741,6 +742,10 @@ struct W8tChoice {
     size_t need = 0;  // bytes of partials with which the same split is chosen (any row tile fits them)
 };
 
+// A plan counts in int: its units are at most kW8tMaxSplits per 64 x 256 tile.
+bool w8t_counts_fit(int M, int N) {
+    return M <= w8p_max_rows() && ((M + 63LL) / 64) * ((N + kPBN - 1LL) / kPBN) <= INT_MAX / kW8tMaxSplits;
+}
 W8tPlan w8t_plan(int M, int N, int it, int S, bool tail) {
     W8tPlan p{};
     p.tiles_m = (M + 64 * it - 1) / (64 * it);
@@ -836,14 +841,14 @@ hipError_t w8t_run_it(const W8tChoice &c, const uint16_t *x, int ldx, const int8
 }  // namespace
 
 size_t w8p_part_bytes(int seq_rows, int max_rows, int N, int K) {
+    if (!w8t_counts_fit(max_rows, N)) return 0;  // no such launch
     return w8t_choose(max_rows, seq_rows, max_rows, N, K, K, kW8tPartBytes).need;
 }
 
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
                       int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st) {
     if (M <= 0) return hipSuccess;
-    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 || M > w8p_max_rows() ||
-        seq_rows <= 0 || seq_rows > M || max_rows < M ||
+    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 || seq_rows <= 0 || seq_rows > M || max_rows < M || !w8t_counts_fit(max_rows, N) ||
         (uint64_t)8 * ldx * 2 >= (1ull << 32) || (uintptr_t)part % 16 ||
         (out.mode != kW8Segments && out.mode != kW8SwiGLU) || (out.mode == kW8SwiGLU && (N % 16 || !out.x16)) ||
         (out.mode == kW8Segments && (out.nseg < 1 || out.nseg > kW8MaxSegs)) ||

@@ -813,19 +813,18 @@ static size_t w8f_ws_bytes(int M, int N, int K) {
     return part ? (part * sizeof(float) + (size_t)(N / 64) * sizeof(uint32_t) + 255) / 256 * 256 : 0;
 }
 
-// M > 16 (the many-row GEMM): [kW8pWsSkip][k-split partials][N / 64 words].
-// The partials start past everything the M <= 16 forms keep in a workspace
+// M > 16 (the many-row GEMM): [kW8pWsSkip][k-split partials].  The partials
+// start past everything an M <= 16 call of any matrix keeps in a workspace
 // (w8f_shape splits fewer than 160 groups at most 32 ways: under 160 * 32 *
-// 64 * 16 floats), and the last words are left alone, so that a workspace
-// whose counters are zero keeps them so.
+// 64 * 16 floats, then under 160 counters), so that one workspace, whose
+// counters have to stay zero, can serve both and several matrices.
 static constexpr size_t kW8pWsSkip = (size_t)160 * 32 * 64 * 16 * sizeof(float) + 4096;
-static size_t w8p_ws_tail(int N) { return ((size_t)(N / 64) * sizeof(uint32_t) + 255) / 256 * 256; }
 
 extern "C" size_t kai_gdn_w8a16_gemm_tiled_workspace_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || N % 64 || K % 256) return 0;
     if (M <= 16) return w8f_ws_bytes(M, N, K);
     const size_t part = gdn::w8p_part_bytes(M, M, N, K);
-    return part ? kW8pWsSkip + part + w8p_ws_tail(N) : 0;
+    return part ? kW8pWsSkip + part : 0;
 }
 
 extern "C" int kai_run_gdn_w8a16_gemm_tiled_hip(const uint16_t *x, const int8_t *Wt, const float *scale, float *y,
@@ -841,11 +840,10 @@ extern "C" int kai_run_gdn_w8a16_gemm_tiled_hip(const uint16_t *x, const int8_t 
         o.seg[0] = gdn::W8Seg{y, N, N};
         o.nseg = 1;
         o.mode = gdn::kW8Segments;
-        const size_t keep = kW8pWsSkip + w8p_ws_tail(N);
-        const bool ws = workspace && aligned(workspace, 16) && workspace_bytes > keep;
+        const bool ws = workspace && aligned(workspace, 16) && workspace_bytes > kW8pWsSkip;
         return (int)gdn::launch_w8p(x, K, Wt, scale, M, M, M, N, K, o,
                                     ws ? reinterpret_cast<float *>(static_cast<char *>(workspace) + kW8pWsSkip) : nullptr,
-                                    ws ? workspace_bytes - keep : 0, (hipStream_t)stream);
+                                    ws ? workspace_bytes - kW8pWsSkip : 0, (hipStream_t)stream);
     }
     const size_t need = w8f_ws_bytes(M, N, K);
     if (need && (!workspace || workspace_bytes < need || !aligned(workspace, 256))) return (int)hipErrorInvalidValue;

@@ -173,3 +173,17 @@ def test_prefill_workspace_query_needs_no_device():
     assert L.kai_gdn_hip_prefill_workspace_bytes(1, 16384, 4) == 23 * 4 * slot
     for bad in ((0, 16384, 32), (1, 0, 32), (1, 16384, 0), (-1, 16384, 32)):
         assert L.kai_gdn_hip_prefill_workspace_bytes(*bad) == 0
+
+
+def test_tiled_gemm_workspace_query():
+    """No bytes for more rows than a call takes (65535 blocks of 256), however
+    large; and what M <= 16 calls keep in a workspace ends before the
+    partial sums of M > 16 calls begin, whatever their matrices."""
+    import orionsbelt_amd as ob
+    need = ob.lib().kai_gdn_w8a16_gemm_tiled_workspace_bytes
+    assert need(333, 2560, 9216) > 0
+    for M, N, K in [(16776961, 2560, 2560), (1354183762, 11392, 25600), (1818695072, 6016, 2048), (818522095, 384, 25600),
+                    (1935160692, 1794791936, 4096), (64713330, 54644608, 9216), (16776960, 2 ** 31 - 64, 4096)]:
+        assert need(M, N, K) == 0, (M, N, K)
+    begin = 160 * 32 * 64 * 16 * 4 + 4096
+    assert max(need(16, 64 * g, 256 * k) for g in range(1, 200) for k in (1, 2, 3, 4, 5, 7, 8, 10, 16, 23, 29, 36, 37, 62, 64)) <= begin
