@@ -746,6 +746,9 @@ struct W8tChoice {
 bool w8t_counts_fit(int M, int N) {
     return M <= w8p_max_rows() && ((M + 63LL) / 64) * ((N + kPBN - 1LL) / kPBN) <= INT_MAX / kW8tMaxSplits;
 }
+// Rows that the 32-bit offsets of a wave's DMA reach (its last 16-byte piece
+// lies 112 bytes into a 64-k step); a wave of a 64 IT-row tile takes 8 IT.
+long long w8t_wave_rows(int ldx) { return ((1LL << 32) - 113) / (2LL * ldx) + 1; }
 W8tPlan w8t_plan(int M, int N, int it, int S, bool tail) {
     W8tPlan p{};
     p.tiles_m = (M + 64 * it - 1) / (64 * it);
@@ -790,7 +793,7 @@ W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, s
     const int ksteps = K / 64;
     const bool tail = seq_rows >= kW8tTailRows;
     part_limit = std::min(part_limit, kW8tPartBytes);
-    const auto it_fits = [&](int it) { return (uint64_t)(8 * it) * ldx * 2 < (1ull << 32); };  // 32-bit row offsets
+    const auto it_fits = [&](int it) { return std::min(8 * it, M) <= w8t_wave_rows(ldx); };
     int S = 1;
     size_t need = 0;
     double best = 1e30;
@@ -842,18 +845,32 @@ hipError_t w8t_run_it(const W8tChoice &c, const uint16_t *x, int ldx, const int8
 
 size_t w8p_part_bytes(int seq_rows, int max_rows, int N, int K) {
     if (!w8t_counts_fit(max_rows, N)) return 0;  // no such launch
+    if (const int reach = (int)std::min(8LL, w8t_wave_rows(K)); reach < std::min(8, max_rows)) seq_rows = max_rows = reach;
     return w8t_choose(max_rows, seq_rows, max_rows, N, K, K, kW8tPartBytes).need;
 }
 
 hipError_t launch_w8p(const uint16_t *x, int ldx, const int8_t *W, const float *scale, int M, int seq_rows,
                       int max_rows, int N, int K, const W8Out &out, float *part, size_t part_bytes, hipStream_t st) {
     if (M <= 0) return hipSuccess;
-    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 || seq_rows <= 0 || seq_rows > M || max_rows < M || !w8t_counts_fit(max_rows, N) ||
-        (uint64_t)8 * ldx * 2 >= (1ull << 32) || (uintptr_t)part % 16 ||
+    if (N <= 0 || N % 64 || K <= 0 || K % 64 || ldx < K || ldx % 8 || (uintptr_t)x % 16 || seq_rows <= 0 || seq_rows > M || max_rows < M || !w8t_counts_fit(max_rows, N) || (uintptr_t)part % 16 ||
         (out.mode != kW8Segments && out.mode != kW8SwiGLU) || (out.mode == kW8SwiGLU && (N % 16 || !out.x16)) ||
         (out.mode == kW8Segments && (out.nseg < 1 || out.nseg > kW8MaxSegs)) ||
         (out.add_in && (out.mode != kW8Segments || out.nseg != 1)))
         return hipErrorInvalidValue;
+    // rows of more than 306 million values: as many at a time as a wave reaches
+    if (const long long reach = w8t_wave_rows(ldx); reach < std::min(8, M)) {
+        for (int m = 0; m < M; m += (int)reach) {
+            const int n = std::min((int)reach, M - m);
+            W8Out o = out;
+            for (W8Seg &sg : o.seg)
+                if (sg.dst) sg.dst += (size_t)m * sg.ld;
+            if (o.x16) o.x16 += (size_t)m * (N / 2);
+            if (o.add_in) o.add_in += (size_t)m * o.add_ld;
+            const hipError_t e = launch_w8p(x + (size_t)m * ldx, ldx, W, scale, n, n, n, N, K, o, part, part_bytes, st);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     const W8tChoice c = w8t_choose(M, seq_rows, max_rows, N, K, ldx, part ? part_bytes : 0);
     if (out.mode == kW8SwiGLU) return w8t_run_it<kW8tSwiGLU>(c, x, ldx, W, scale, M, N, K, part, out, st);
     if (out.add_in) return w8t_run_it<kW8tAdd>(c, x, ldx, W, scale, M, N, K, part, out, st);

@@ -172,6 +172,33 @@ def test_w8a16_gemm_many_rows_workspaces(L, M, N, K):
     assert torch.equal(y8, small())
 
 
+def test_w8a16_gemm_many_rows_longest_rows(L):
+    """Rows too long for the 32-bit offsets of eight of them (K over 306
+    million): seven at a time.  A few nonzero activations, so that the sums
+    are exact."""
+    torch = torch_mod()
+    M, N, K = 17, 64, 306783744
+    assert 7 * K * 2 + 112 >= 2 ** 32 > 6 * K * 2 + 112
+    w = torch.randint(-127, 128, (N, K), device="cuda", dtype=torch.int8)
+    wt = torch.empty_like(w)
+    assert L.kai_run_gdn_w8_tile_hip(P(w), P(wt), N, K, stream()) == 0
+    x = torch.zeros(M, K, dtype=torch.float16, device="cuda")
+    ref = torch.zeros(M, N, dtype=torch.float64, device="cuda")
+    for m in range(M):
+        for k in (0, 63 * m + 5, K // 2 + 129 * m, K - 1 - m):
+            x[m, k] = m + 1
+            ref[m] += (m + 1) * w[:, k].double()
+    del w
+    sc = torch.ones(N, device="cuda")
+    nb = L.kai_gdn_w8a16_gemm_tiled_workspace_bytes(M, N, K)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device="cuda")
+    y = torch.full((M, N), float("nan"), device="cuda")
+    assert L.kai_run_gdn_w8a16_gemm_tiled_hip(P(x), P(wt), P(sc), P(y), M, N, K, P(ws), nb, stream()) == 0
+    assert torch.equal(y.double(), ref)
+    del x, wt
+    torch.cuda.empty_cache()
+
+
 def test_w8a16_gemm_tiled_rejects_bad_args(L):
     torch = torch_mod()
     t = empty((16 * 4096,), torch.float32)
