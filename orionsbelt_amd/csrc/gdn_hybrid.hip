@@ -869,10 +869,6 @@ hipError_t step(kai_gdn_hybrid *m, const int32_t *tokens, int32_t *next, float *
 // group: at a few hundred rows a launch's time hardly depends on the rows
 // (four 200-token prompts of the 4B model: 42 ms one after another).
 constexpr int kPrefillGroupRows = 4096;
-// Longest prompt (chunks of 64) the chunked delta rule runs as one segment
-// whatever the batch; longer ones run one sequence per call, so that their
-// segments, and with them their roundings, do not depend on the batch.
-constexpr int kPrefillGroupChunks = 11;
 
 // Sequences of T rows that run as one group at most (whatever the batch).
 int group_limit(const kai_gdn_hybrid *m, int T) {
@@ -1001,7 +997,9 @@ hipError_t prefill_group(kai_gdn_hybrid *m, const int32_t *tokens, int b0, Rows 
             const size_t s1 = (size_t)Hv * 128 * 128;
             float *S = L.S + b0 * s1;
             TRY(hipMemsetAsync(S, 0, r.nseq * s1 * sizeof(float), st));
-            const int together = (T + 63) / 64 <= kPrefillGroupChunks ? r.nseq : 1;
+            // one sequence per call where the segments, and with them the
+            // roundings, would depend on the batch
+            const int together = (T + 63) / 64 <= prefill_one_segment_chunks() ? r.nseq : 1;
             for (int i = 0; i < r.nseq; i += together) {
                 const size_t t0 = (size_t)i * T;
                 const int rc = kai_run_gdn_chunk_delta_rule_bf16_f32_hip(

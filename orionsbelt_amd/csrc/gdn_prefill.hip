@@ -1649,6 +1649,7 @@ __global__ __launch_bounds__(NT) void prefill_pass2_kernel(SegArgs a) {
 // 56.6 us, 2K: 68.7 against 77.9 us, 4K: 93.1 against 94.5 us; 3 is as good
 // at 1K and worse at 2K)
 constexpr int kMinSegChunks = 4;
+constexpr int kMinSegs = 3;  // the fewest segments of a plan that has any
 constexpr int kTargetWgs = 256;
 constexpr double kCostTrans = 1.10, kCostStep = 1.26, kCostPrologue = 1.0;
 
@@ -1723,7 +1724,7 @@ void plan_segments(int B, int Hv, int NC, SegPlan &pl) {
     int best[kMaxSegs], len[kMaxSegs];
     double best_cost = (double)NC;  // one segment: the plain recurrence
     int best_p = 1;
-    for (int P = 3; P <= pmax; ++P) {
+    for (int P = kMinSegs; P <= pmax; ++P) {
         const double cost = plan_lengths(P, NC, len);
         if (cost < best_cost) {
             best_cost = cost;
@@ -1811,6 +1812,8 @@ LastWindowCall *last_window_slot() {
 }
 
 }  // namespace
+
+int prefill_one_segment_chunks() { return kMinSegs * kMinSegChunks - 1; }
 
 size_t prefill_carry_bytes(int B, int T, int Hv) {
     const int NC = (T + C - 1) / C;

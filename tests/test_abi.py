@@ -187,3 +187,16 @@ def test_tiled_gemm_workspace_query():
         assert need(M, N, K) == 0, (M, N, K)
     begin = 160 * 32 * 64 * 16 * 4 + 4096
     assert max(need(16, 64 * g, 256 * k) for g in range(1, 200) for k in (1, 2, 3, 4, 5, 7, 8, 10, 16, 23, 29, 36, 37, 62, 64)) <= begin
+
+
+def test_one_segment_limit_follows_the_planner():
+    """The model groups prompts up to gdn::prefill_one_segment_chunks(); no
+    batch and head count may be planned in segments up to there (a segmented
+    plan has a carry buffer), and one chunk more is planned for some."""
+    import orionsbelt_amd as ob
+    L = ob.lib()
+    chunks = L._ZN3gdn26prefill_one_segment_chunksEv()
+    need = L.kai_gdn_hip_prefill_workspace_bytes
+    heads = (1, 2, 4, 8, 16, 32, 64)
+    assert not any(need(b, 64 * n, h) for b in range(1, 17) for n in range(1, chunks + 1) for h in heads)
+    assert any(need(1, 64 * chunks + 1, h) for h in heads)
