@@ -50,11 +50,15 @@ template <int N> GDN_DEV void wait_vm() { __builtin_amdgcn_s_waitcnt((N & 15) | 
 // Written as asm so that the compiler does not count it against the LDS reads
 // of the other ring slots (it would wait for every DMA before them); the
 // kernel's own wait_vm and barriers order it.  The compiler does not see that
-// the asm reads base in a vector memory operation: base must come from scalar
-// arithmetic, not straight from a readfirstlane (five wait states apart).
+// the asm reads base in a vector memory operation, which takes five wait
+// states after a readfirstlane: base is derived by scalar arithmetic from what
+// dma_bases returned.  (With the wait states in here the GEMM is 3% slower.)
 GDN_DEV void dma16(const void *base, uint32_t off, uint32_t lds) {
     __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-                     : "memory");
+                     : "memory", "m0");
+}
+template <typename A, typename B> GDN_DEV void dma_bases(const A *&a, const B *&b) {
+    __asm__ volatile("s_nop 4" : "+s"(a), "+s"(b));
 }
 GDN_DEV int scalar(int x) { return __builtin_amdgcn_readfirstlane(x); }
 GDN_DEV uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(const lds_void_t *)p; }
@@ -293,7 +297,7 @@ __device__ __forceinline__ void w8t_body(const uint16_t *__restrict__ X, int ldx
         const int r0 = min(t.m0 + 8 * IT * wave, M - 1);  // the wave's first row
         xnext = X + (size_t)scalar(r0) * ldx + (size_t)scalar(t.s0) * 64;
         wnext = W + ((size_t)scalar(wg) * ksteps + scalar(t.s0)) * 4096 + (2 * wave & 3) * 1024;
-        __asm__ volatile("s_nop 4" : "+s"(xnext), "+s"(wnext));  // see dma16
+        dma_bases(xnext, wnext);
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
             const int row = 8 * i + (lane >> 3);  // of the wave's 8 IT
@@ -590,9 +594,10 @@ __global__ __launch_bounds__(kApThreads) void attn_prefill_kernel(
     auto dma = [&](int kb, int b) {
         const int t0 = min(kb * kApK + 16 * (wave >> 1), Tmax - 16);
         const uint16_t *kp = kbase + (size_t)t0 * kApD + (4 * (wave & 1)) * 512;
+        const uint16_t *vp = vbase + (size_t)(32 * wave) * Tv + kb * kApK;
+        dma_bases(kp, vp);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dma16(kp + i * 512, koff, kl + 32768u * b + 1024u * i);
-        const uint16_t *vp = vbase + (size_t)(32 * wave) * Tv + kb * kApK;
 #pragma unroll
         for (int i = 0; i < 4; ++i) dma16(vp + (size_t)(8 * i) * Tv, voff, vl + 32768u * b + 1024u * i);
     };
