@@ -293,7 +293,11 @@ int kai_run_gdn_w8a16_gemm_hip(const uint16_t *x, const int8_t *Wq, const float 
  * 256 x 256 output tiles).  Its workspace is optional and needs no zeroing:
  * with the bytes that the query returns, few rows split k across blocks
  * (summed in a fixed order); with less, or none, they split less or not at
- * all.  It changes nothing of a workspace that a call with M <= 16 keeps. */
+ * all.  So for M > 16 the order of a row's sum, and with it its last bits,
+ * follows from M, N, K and the workspace's size (calls alike in these give
+ * the same bits); every split's result is within the fp32 sum's rounding.
+ * Calls that use one workspace must not overlap.  It changes nothing of a
+ * workspace that a call with M <= 16 keeps. */
 int kai_run_gdn_w8_tile_hip(const int8_t *Wq, int8_t *Wt, int N, int K, void *stream);
 size_t kai_gdn_w8a16_gemm_tiled_workspace_bytes(int M, int N, int K);
 int kai_run_gdn_w8a16_gemm_tiled_hip(const uint16_t *x, const int8_t *Wt, const float *scale,
@@ -315,7 +319,10 @@ int kai_run_gdn_w8_quantize_hip(const float *W, int8_t *Wq, float *scale, int N,
  * fp32.  num_q_heads / num_kv_heads <= 4.  `workspace` should hold
  * kai_gdn_attn_decode_workspace_bytes(batch, num_q_heads, length) bytes; the
  * least accepted is 1032 bytes per sequence, query head and 256 positions (a
- * part counts whole), with which short contexts are split less and run slower. */
+ * part counts whole), with which short contexts are split less and run slower.
+ * The positions are split by batch, num_kv_heads, length and workspace_bytes:
+ * a sequence's last bits depend on these (calls alike in them give the same
+ * bits), not on its own length alone. */
 size_t kai_gdn_attn_decode_workspace_bytes(int batch, int num_q_heads, int length);
 int kai_run_gdn_attn_decode_f16kv_hip(const uint16_t *q, const uint16_t *k_cache,
                                       const uint16_t *v_cache, float *out, int batch,

@@ -193,7 +193,8 @@ GDN_DEV void w8t_epilogue(const f32x16_t (&acc)[IT][2], float *scratch, int row0
 // of K; from there, part (u - full) % S of the k-steps of tile full +
 // (u - full) / S, its sums going to `part` unscaled for w8t_reduce_kernel.
 // Blocks take units blockIdx, blockIdx + grid, ...; unit u runs on XCD u % 8
-// (blocks are handed out round robin and the grid is a multiple of 8).
+// (blocks are handed out round robin; the grid is 256, or, below 256 units,
+// the unit count, and then no block takes a second one).
 struct W8tPlan {
     int tiles_m, tiles_n, full, S, units, grid;
 };
@@ -790,10 +791,15 @@ double w8t_cost(const W8tPlan &p, int it, int ksteps) {
 // The row tile (64 IT) and the k-splits of M rows made of sequences of
 // `seq_rows` rows each, at most max_rows together.  The split decides the
 // order of a sum, so it is chosen without M (a sequence's result does not
-// depend on how many sequences it is batched with); the row tile does not
-// change a bit and is chosen for M.  Below kW8tTailRows every tile is split alike; from
-// there (where a launch holds one sequence) only the tiles left over after
-// the whole rounds of 256.
+// depend on how many sequences it is batched with).  Its price: a group whose
+// tiles fill the chip still writes and sums the parts that one of its
+// sequences alone wants (16 prompts of 200 rows through the 4B model 31 ms,
+// modelled 25 without; one after another, each as its own launch, 172).
+// Below kW8tTailRows every tile is split alike, the row tile does not change a
+// bit, and it is chosen for M.  From there (where a launch holds one sequence)
+// only the tiles left over after the whole rounds of 256 are split: the row
+// tile decides which rows those are, and it is the one that the split was
+// chosen with.
 W8tChoice w8t_choose(int M, int seq_rows, int max_rows, int N, int K, int ldx, size_t part_limit) {
     const int ksteps = K / 64;
     const bool tail = seq_rows >= kW8tTailRows;
